@@ -1869,10 +1869,20 @@ __device__ inline void wave_lds_sync() {
 // accumulation order is fixed; codes are distinct (a supervoxel lists a
 // Gaussian at most once). The first nshort blocks take 16 Gaussians each, 16
 // lanes per Gaussian: a bitonic sort in LDS over the next power of two, for
-// lists up to kSortShort. The kSortLongBlocks blocks after them take the
-// Gaussians with longer lists (listed by the pair scan), one at a time: a
-// bitonic sort in LDS, or a block-wide rank sort beyond kSortLds entries.
-constexpr int kSortLongBlocks = 64;
+// lists up to kSortShort. The nlong blocks after them take the Gaussians
+// with longer lists (listed by the pair scan), one at a time: a bitonic sort
+// in LDS, or a block-wide rank sort beyond kSortLds entries.
+// A long list is a chain of barriers and LDS round trips (about 20 us for 512
+// entries alone on a CU), so what bounds the long lists is how many are
+// sorted at once: nlong is 64 where few lists are long, and enough to fill
+// the chip (8 blocks on each CU, by threads) where the lists average 64
+// entries or more (every list of a per-voxel frame). Per-voxel frame of 4.9M
+// voxels and 10,000 Gaussians: 3157 us with 64 blocks, 156 us with 2048.
+constexpr int kSortLongFew = 64;
+constexpr int kSortLongMany = 2048;
+inline int sort_long_blocks(const DevPtrs& P) {
+  return P.Sext >= 64 * P.Gext ? (int)std::min<long long>(P.Gext, kSortLongMany) : kSortLongFew;
+}
 
 __device__ inline void seg_sort_short(const DevPtrs& P, int* sh) {
   const int grp = threadIdx.x >> 4, lane = threadIdx.x & 15;
@@ -1910,9 +1920,9 @@ __device__ inline void seg_sort_short(const DevPtrs& P, int* sh) {
   for (int i = lane; i < L; i += 16) P.pairs_sorted[st + i] = a[i];
 }
 
-__device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first) {
+__device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int nlong) {
   const int cnt = P.knn_ctl[2];
-  for (int li = first; li < cnt; li += kSortLongBlocks) {
+  for (int li = first; li < cnt; li += nlong) {
     const long long k = P.long_list[li];
     const int st = P.seg_start[k], L = P.seg_start[k + 1] - st;
     const int t = threadIdx.x;
@@ -1929,31 +1939,38 @@ __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first) {
     while (n < L) n <<= 1;
     for (int i = t; i < n; i += 256) sh[i] = i < L ? P.pairs[st + i] : INT_MAX;
     __syncthreads();
+    // pairs (lo, lo + j) as in the short sort, pair i at thread i mod 256: in
+    // a step with j <= 64 a wave's 64 pairs are 128 consecutive entries, so
+    // only its own lanes' accesses have to be ordered between two such steps
+    int pj = 0;
     for (int w = 2; w <= n; w <<= 1)
       for (int j = w >> 1; j > 0; j >>= 1) {
-        for (int i = t; i < n; i += 256) {
-          const int p = i ^ j;
-          if (p > i) {
-            const int a = sh[i], b = sh[p];
-            if ((a > b) == ((i & w) == 0)) {
-              sh[i] = b;
-              sh[p] = a;
-            }
+        if (j > 64 || pj > 64)
+          __syncthreads();
+        else
+          wave_lds_sync();
+        for (int i = t; i < (n >> 1); i += 256) {
+          const int lo = 2 * i - (i & (j - 1)), hi = lo + j;
+          const int x = sh[lo], y = sh[hi];
+          if ((x > y) == ((lo & w) == 0)) {
+            sh[lo] = y;
+            sh[hi] = x;
           }
         }
-        __syncthreads();
+        pj = j;
       }
+    __syncthreads();
     for (int i = t; i < L; i += 256) P.pairs_sorted[st + i] = sh[i];
     __syncthreads();  // sh is free for the next list
   }
 }
 
-__global__ __launch_bounds__(256) void k_seg_sort(DevPtrs P, int nshort) {
+__global__ __launch_bounds__(256) void k_seg_sort(DevPtrs P, int nshort, int nlong) {
   __shared__ int sh[kSortLds > 16 * kSortShort ? kSortLds : 16 * kSortShort];
   if ((int)blockIdx.x < nshort)
     seg_sort_short(P, sh);
   else
-    seg_sort_long(P, sh, (int)blockIdx.x - nshort);
+    seg_sort_long(P, sh, (int)blockIdx.x - nshort, nlong);
 }
 
 // Posterior (GMEM.cu:1601-1677) and regularisation (GMEM.cu:1693-1809) of
@@ -2961,7 +2978,8 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
   if (tk == TK_ESTEP && e1) (void)hipEventRecord(e1, st);
   k_scan_frames<<<P.nframes, 1024, 0, st>>>(P, 1, 1, O.K);
   k_pair_scatter<KM><<<nb(P.Sext, bs), bs, 0, st>>>(P, O);
-  k_seg_sort<<<nb(P.Gext, 16) + kSortLongBlocks, 256, 0, st>>>(P, (int)nb(P.Gext, 16));
+  const int nlong = sort_long_blocks(P);
+  k_seg_sort<<<nb(P.Gext, 16) + nlong, 256, 0, st>>>(P, (int)nb(P.Gext, 16), nlong);
   if (tk == TK_MSTEP && e0) (void)hipEventRecord(e0, st);
   launch_mstep(P, O, st);
   if (tk == TK_MSTEP && e1) (void)hipEventRecord(e1, st);
