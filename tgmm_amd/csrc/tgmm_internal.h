@@ -148,8 +148,11 @@ struct DevPtrs {
   // M-step segments
   int* seg_cnt;     // Gcap+1
   int* seg_start;   // Gcap+1
-  int* pairs;       // K*Scap
-  int* pairs_sorted;
+  int* run_cnt;     // Gcap: pair runs listed so far (zero between iterations)
+  int* pairs;       // K*Scap: each Gaussian's runs of pairs, unordered, from its
+                    // segment's start: the code of a run's first pair
+  unsigned char* run_len;  // K*Scap: pairs of each run, 1..64
+  int* pairs_sorted;  // K*Scap: each Gaussian's pairs, ordered by supervoxel
   // grid
   int* cell_cnt;    // Ccap+1
   int* cell_start;  // Ccap+1

@@ -425,7 +425,7 @@ __global__ __launch_bounds__(kGB) void k_alpha_init(DevPtrs P) {
 }
 
 // ---------------------------------------------------------------- scans --
-constexpr int kSortShort = 128;  // longer pair lists are sorted by a block each
+constexpr int kSortShort = 128;  // longer pair lists are listed for the block-wide sort
 constexpr int kScanQ = 8;        // int4 loads per thread and pass, k_scan_frames (4 | kScanQ)
 constexpr int kSortLds = 4096;   // longest list sorted in LDS
 
@@ -1814,13 +1814,18 @@ __global__ __launch_bounds__(256) void k_estep(DevPtrs P, KOpts O) {
   estep_one<KM>(P, O, s, ok);
 }
 
-// Each significant pair's code at its Gaussian's list, in a slot taken from
-// the count (the lists are ordered by k_seg_sort). The candidates' indices
-// and responsibilities depend on s alone (s < Scap) and are loaded before the
-// frame checks; the slot reservations of all candidates are issued back to
-// back and their results used after, so that a wave waits for one round of
-// atomics, not K. Branch-free over the candidates (slots j >= K read row 0
-// and hold no pair), so that no wait is forced at branch joins.
+// Each run of significant pairs (consecutive lanes of a wave, one Gaussian,
+// one slot j: supervoxels s, s+1, ... ) as one entry of its Gaussian's list:
+// the code of its first pair and its length, in an entry taken from run_cnt
+// (k_seg_sort orders the runs and writes the pairs out): few entries to order.
+// This kernel's own time is the reads of ind and rnk (13 us at 60,000
+// Gaussians, 101 us on a per-voxel frame of 4.9M voxels, as with an entry per
+// pair). The candidates' indices and
+// responsibilities depend on s alone (s < Scap) and are loaded before the
+// frame checks; the entries of all candidates are reserved back to back and
+// used after, so that a wave waits for one round of atomics, not K.
+// Branch-free over the candidates (slots j >= K read row 0 and hold no pair),
+// so that no wait is forced at branch joins.
 template <int KM>
 __global__ __launch_bounds__(256) void k_pair_scatter(DevPtrs P, KOpts O) {
   const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1836,25 +1841,26 @@ __global__ __launch_bounds__(256) void k_pair_scatter(DevPtrs P, KOpts O) {
     rr[j] = P.rnk[row * S + s];
   }
   const int f = P.sblk_frame[s >> 8];
-  // no early exit: every lane takes part in the wave-wide slot reservation
+  // no early exit: every lane takes part in the wave-wide runs
   const bool ok = f >= 0 && P.fr[f].active && P.sv_frame[s] == f;
-  int key[KM], head[KM], old[KM], st[KM];
+  int len[KM], slot[KM], st[KM];
 #pragma unroll
   for (int j = 0; j < KM; j++) {
-    key[j] = (j < K && ok && kr[j] >= 0 && pair_significant(rr[j])) ? kr[j] : -1;
-    const WaveRun r = wave_run(key[j]);
-    head[j] = r.head;
+    const int key = (j < K && ok && kr[j] >= 0 && pair_significant(rr[j])) ? kr[j] : -1;
+    const WaveRun r = wave_run(key);
+    const bool head = key >= 0 && r.head == lane;
+    len[j] = head ? r.len : 0;
     int o = 0;
-    if (key[j] >= 0 && r.head == lane) o = atomicSub(P.seg_cnt + key[j], r.len);
-    old[j] = o;
-    st[j] = P.seg_start[key[j] >= 0 ? key[j] : 0];
+    if (head) o = atomicAdd(P.run_cnt + key, 1);
+    slot[j] = o;
+    st[j] = P.seg_start[head ? key : 0];
   }
 #pragma unroll
   for (int j = 0; j < KM; j++) {
-    // a run of lanes with one key takes the slots below the value its head
-    // took, counting down in lane order
-    const int o = __shfl(old[j], head[j], 64);
-    if (key[j] >= 0) P.pairs[st[j] + o - 1 - (lane - head[j])] = (int)((s << kPairShift) | j);
+    if (len[j] > 0) {
+      P.pairs[st[j] + slot[j]] = (int)((s << kPairShift) | j);
+      P.run_len[st[j] + slot[j]] = (unsigned char)len[j];
+    }
   }
 }
 
@@ -1865,19 +1871,27 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Pair lists ordered by code (= by supervoxel), so that the FP64
-// accumulation order is fixed; codes are distinct (a supervoxel lists a
-// Gaussian at most once). The first nshort blocks take 16 Gaussians each, 16
-// lanes per Gaussian: a bitonic sort in LDS over the next power of two, for
-// lists up to kSortShort. The nlong blocks after them take the Gaussians
-// with longer lists (listed by the pair scan), one at a time: a bitonic sort
-// in LDS, or a block-wide rank sort beyond kSortLds entries.
-// A long list is a chain of barriers and LDS round trips (about 20 us for 512
-// entries alone on a CU), so what bounds the long lists is how many are
-// sorted at once: nlong is 64 where few lists are long, and enough to fill
-// the chip (8 blocks on each CU, by threads) where the lists average 64
-// entries or more (every list of a per-voxel frame). Per-voxel frame of 4.9M
-// voxels and 10,000 Gaussians: 3157 us with 64 blocks, 156 us with 2048.
+// Pair lists written out in order of code (= of supervoxel), so that the FP64
+// accumulation order is fixed. A Gaussian's runs (k_pair_scatter) hold
+// disjoint ranges of supervoxels (a supervoxel lists a Gaussian at most
+// once), so a run's place is the sum of the lengths of the runs with a
+// smaller first code, and its pairs follow each other: no pair is compared.
+// The first nshort blocks take 16 Gaussians each, 16 lanes per Gaussian with
+// up to 16 runs (a run a lane, compared by shuffles) or up to kSortShort pairs
+// (in LDS). The nlong blocks after them take the Gaussians with more of both,
+// one at a time, among those with more than kSortShort pairs (listed by the
+// pair scan): up to kRunLds runs ranked in LDS, a run a thread; beyond, the
+// pairs laid out and sorted in LDS (bitonic), or, past kSortLds pairs, the
+// runs ranked from memory. Both sides read the run count; whichever handles a
+// Gaussian clears it (the other, reading 0, writes nothing).
+// Latency-bound. Against sorting the pairs themselves: 60,000 Gaussians 22.4
+// -> 12.5 us, 200 Gaussians 5.1 -> 3.6 us, per-voxel frames of 4.9M and 40,000
+// voxels 156 -> 49.5 and 19.5 -> 9.5 us.
+// nlong is 64 where few lists are long, and enough to fill the chip (8 blocks
+// on each CU, by threads) where the lists average 64 pairs or more: a long
+// list is a chain of barriers and LDS round trips (about 20 us for 512 pairs),
+// and lists of scattered voxels have as many runs as pairs.
+constexpr int kRunLds = 512;
 constexpr int kSortLongFew = 64;
 constexpr int kSortLongMany = 2048;
 inline int sort_long_blocks(const DevPtrs& P) {
@@ -1890,58 +1904,128 @@ __device__ inline void seg_sort_short(const DevPtrs& P, int* sh) {
   // the list's bounds and the Gaussian's frame are in range for every k <
   // Gext; they are loaded before the frame checks, used only after them
   const int gf = P.g_frame[k];
-  const int st = P.seg_start[k], en = P.seg_start[k + 1];
+  const int st = P.seg_start[k], L = P.seg_start[k + 1] - st;
+  const int nr = P.run_cnt[k];
   const int f = P.gblk_frame[k / kGB];
   if (f < 0 || !P.fr[f].active) return;
   if (gf != f) return;
-  const int L = en - st;
-  if (L <= 1 || L > kSortShort) {
-    if (L == 1 && lane == 0) P.pairs_sorted[st] = P.pairs[st];
+  if (lane == 0) P.seg_cnt[k] = 0;  // the counts of the next iteration
+  if (nr <= 0 || (nr > 16 && L > kSortShort)) return;
+  if (lane == 0) P.run_cnt[k] = 0;
+  if (nr <= 16) {
+    const int c = lane < nr ? P.pairs[st + lane] : INT_MAX;
+    const int n = lane < nr ? P.run_len[st + lane] : 0;
+    int at = 0;
+    for (int i = 0; i < nr; i++) {
+      const int ci = __shfl(c, i, 16), ni = __shfl(n, i, 16);
+      at += ci < c ? ni : 0;
+    }
+    for (int i = 0; i < nr; i++) {
+      const int ci = __shfl(c, i, 16), ni = __shfl(n, i, 16), ai = __shfl(at, i, 16);
+      for (int t = lane; t < ni; t += 16)
+        P.pairs_sorted[st + ai + t] = ci + (t << kPairShift);
+    }
     return;
   }
-  int* a = sh + grp * kSortShort;
-  int n = 2;
-  while (n < L) n <<= 1;
-  for (int i = lane; i < n; i += 16) a[i] = i < L ? P.pairs[st + i] : INT_MAX;
+  int* code = sh + grp * 2 * kSortShort;
+  int* place = code + kSortShort;  // the length, then also the place (above bit 8)
+  for (int i = lane; i < nr; i += 16) {
+    code[i] = P.pairs[st + i];
+    place[i] = P.run_len[st + i];
+  }
   wave_lds_sync();
-  for (int w = 2; w <= n; w <<= 1)
-    for (int j = w >> 1; j > 0; j >>= 1) {
-      // pairs (lo, lo + j) with bit j of lo clear; ascending where bit w is
-      for (int i = lane; i < (n >> 1); i += 16) {
-        const int lo = 2 * i - (i & (j - 1)), hi = lo + j;
-        const int x = a[lo], y = a[hi];
-        if ((x > y) == ((lo & w) == 0)) {
-          a[lo] = y;
-          a[hi] = x;
-        }
-      }
-      wave_lds_sync();
+  int at[kSortShort / 16];
+#pragma unroll
+  for (int q = 0; q < kSortShort / 16; q++) {
+    const int r = lane + 16 * q;
+    at[q] = 0;
+    if (r < nr) {
+      const int c = code[r];
+      for (int i = 0; i < nr; i++) at[q] += code[i] < c ? place[i] : 0;
     }
-  for (int i = lane; i < L; i += 16) P.pairs_sorted[st + i] = a[i];
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int q = 0; q < kSortShort / 16; q++) {
+    const int r = lane + 16 * q;
+    if (r < nr) place[r] |= at[q] << 8;
+  }
+  wave_lds_sync();
+  for (int i = 0; i < nr; i++) {
+    const int c = code[i], n = place[i] & 255, a = place[i] >> 8;
+    for (int t = lane; t < n; t += 16) P.pairs_sorted[st + a + t] = c + (t << kPairShift);
+  }
 }
 
 __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int nlong) {
+  __shared__ int fill;
   const int cnt = P.knn_ctl[2];
   for (int li = first; li < cnt; li += nlong) {
     const long long k = P.long_list[li];
+    const int nr = P.run_cnt[k];
+    if (nr <= 16) continue;  // a count above 16 is cleared by this block alone
     const int st = P.seg_start[k], L = P.seg_start[k + 1] - st;
     const int t = threadIdx.x;
-    if (L > kSortLds) {
-      for (int i = t; i < L; i += 256) {
-        const int e = P.pairs[st + i];
-        int rank = 0;
-        for (int j = 0; j < L; j++) rank += (P.pairs[st + j] < e) ? 1 : 0;
-        P.pairs_sorted[st + rank] = e;
+    if (nr <= kRunLds) {
+      int* code = sh;
+      int* place = sh + kRunLds;
+      for (int r = t; r < nr; r += 256) {
+        code[r] = P.pairs[st + r];
+        place[r] = P.run_len[st + r];
       }
+      __syncthreads();
+      if (t == 0) P.run_cnt[k] = 0;  // read by every thread before the barrier
+      int at[kRunLds / 256];
+#pragma unroll
+      for (int q = 0; q < kRunLds / 256; q++) {
+        const int r = t + 256 * q;
+        at[q] = 0;
+        if (r < nr) {
+          const int c = code[r];
+#pragma unroll 8
+          for (int i = 0; i < nr; i++) at[q] += code[i] < c ? place[i] : 0;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kRunLds / 256; q++) {
+        const int r = t + 256 * q;
+        if (r < nr) place[r] |= at[q] << 7;
+      }
+      __syncthreads();
+      for (int i = t >> 4; i < nr; i += 16) {
+        const int c = code[i], n = place[i] & 127, a = place[i] >> 7;
+        for (int u = t & 15; u < n; u += 16) P.pairs_sorted[st + a + u] = c + (u << kPairShift);
+      }
+      __syncthreads();  // sh is free for the next list
+      continue;
+    }
+    if (L > kSortLds) {
+      for (int r = t; r < nr; r += 256) {
+        const int c = P.pairs[st + r], n = P.run_len[st + r];
+        int at = 0;
+        for (int i = 0; i < nr; i++) at += P.pairs[st + i] < c ? P.run_len[st + i] : 0;
+        for (int u = 0; u < n; u++) P.pairs_sorted[st + at + u] = c + (u << kPairShift);
+      }
+      __syncthreads();  // every thread has read the count
+      if (t == 0) P.run_cnt[k] = 0;
       continue;
     }
     int n = 1;
     while (n < L) n <<= 1;
-    for (int i = t; i < n; i += 256) sh[i] = i < L ? P.pairs[st + i] : INT_MAX;
+    if (t == 0) fill = 0;
+    for (int i = L + t; i < n; i += 256) sh[i] = INT_MAX;
     __syncthreads();
-    // pairs (lo, lo + j) as in the short sort, pair i at thread i mod 256: in
-    // a step with j <= 64 a wave's 64 pairs are 128 consecutive entries, so
-    // only its own lanes' accesses have to be ordered between two such steps
+    if (t == 0) P.run_cnt[k] = 0;  // read by every thread before the barrier
+    for (int r = t; r < nr; r += 256) {
+      const int c = P.pairs[st + r], len = P.run_len[st + r];
+      const int at = atomicAdd(&fill, len);
+      for (int u = 0; u < len; u++) sh[at + u] = c + (u << kPairShift);
+    }
+    __syncthreads();
+    // pairs (lo, lo + j), pair i at thread i mod 256: in a step with j <= 64
+    // a wave's 64 pairs are 128 consecutive entries, so only its own lanes'
+    // accesses have to be ordered between two such steps
     int pj = 0;
     for (int w = 2; w <= n; w <<= 1)
       for (int j = w >> 1; j > 0; j >>= 1) {
@@ -1950,6 +2034,7 @@ __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int n
         else
           wave_lds_sync();
         for (int i = t; i < (n >> 1); i += 256) {
+          // lo has bit j clear; ascending where bit w is
           const int lo = 2 * i - (i & (j - 1)), hi = lo + j;
           const int x = sh[lo], y = sh[hi];
           if ((x > y) == ((lo & w) == 0)) {
@@ -1966,7 +2051,7 @@ __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int n
 }
 
 __global__ __launch_bounds__(256) void k_seg_sort(DevPtrs P, int nshort, int nlong) {
-  __shared__ int sh[kSortLds > 16 * kSortShort ? kSortLds : 16 * kSortShort];
+  __shared__ int sh[kSortLds > 32 * kSortShort ? kSortLds : 32 * kSortShort];
   if ((int)blockIdx.x < nshort)
     seg_sort_short(P, sh);
   else

@@ -110,7 +110,9 @@ int ws_alloc(Workspace* w, const WsShape& sh, int K) {
   AL(P.gblk_frame, G / kGB);
   AL(P.seg_cnt, G + 1);
   AL(P.seg_start, G + 1);
+  AL(P.run_cnt, G);
   AL(P.pairs, (long long)K * S);
+  AL(P.run_len, (long long)K * S);
   AL(P.pairs_sorted, (long long)K * S);
   AL(P.cell_cnt, C + 1);
   AL(P.cell_start, C + 1);
@@ -142,9 +144,9 @@ void ws_free(Workspace* w) {
 
 long long ws_bytes_estimate(const WsShape& sh, int K) {
   const long long S = sh.Scap, G = sh.Gcap, C = sh.Ccap, V = sh.Vcap;
-  return 24 * V + S * (16 + 8 + 4 + 12 + 80 + 80 + 12 + 16 + 16LL * K + 1 + 4 + 8) +
+  return 24 * V + S * (16 + 8 + 4 + 12 + 80 + 80 + 12 + 16 + 17LL * K + 1 + 4 + 8) +
          G * (4 + 8 * GS_NFIELDS * 2 + 1 + 96 + 8 + 64 + 12 + 4 + 8 + 12 + 4 + 1 + 16 + 288 +
-              68 + 4) +
+              68 + 4 + 4) +
          8 * C + 64 * sh.Fcap;
 }
 
@@ -441,6 +443,7 @@ int batch_upload(tgmm_batch* b, const std::vector<FrameSrc>& fs) {
   HIPCHK(hipMemsetAsync(P.ind, 0xFF, (size_t)b->ws.K * S * 4, st));
   HIPCHK(hipMemsetAsync(P.rnk, 0, (size_t)b->ws.K * S * 4, st));
   HIPCHK(hipMemsetAsync(P.seg_cnt, 0, (G + 1) * 4, st));
+  HIPCHK(hipMemsetAsync(P.run_cnt, 0, G * 4, st));
   HIPCHK(hipMemsetAsync(P.cell_cnt, 0, (sh.Ccap + 1) * 4, st));
   HIPCHK(launch_prep(P, b->ko, st));
   b->grid_cell = b->ko.tiles.knn_cell;

@@ -346,6 +346,7 @@ extern "C" int tgmm_server_create(int device, const tgmm_server_opts* opts, tgmm
       (er = hipMemsetAsync(P.ind, 0xFF, (size_t)e.K * S * 4, s->st)) ||
       (er = hipMemsetAsync(P.rnk, 0, (size_t)e.K * S * 4, s->st)) ||
       (er = hipMemsetAsync(P.seg_cnt, 0, (G + 1) * 4, s->st)) ||
+      (er = hipMemsetAsync(P.run_cnt, 0, G * 4, s->st)) ||
       (er = hipMemsetAsync(P.cell_cnt, 0, (sh.Ccap + 1) * 4, s->st)) ||
       (er = hipMemsetAsync(P.knn_ctl, 0, 64 * 4, s->st)) ||
       (er = hipMemsetAsync(P.svkeep, 0, (size_t)17 * G * 4, s->st)) ||
