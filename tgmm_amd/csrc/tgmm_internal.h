@@ -173,6 +173,7 @@ struct DevPtrs {
   // reductions
   double* part_g;   // Gcap/kGB
   double* part_g2;  // Gcap/kGB: sums of alpha after the posterior update (death test)
+  double* mst;      // 10*Gcap: the M-step's sums N, S1[3], S2[6], field-major
   double* part_s;   // Scap/kLLminB: log-likelihood block partials
   double* part_sg;  // Scap/256: partials of 256-supervoxel groups
   FrameDev* fr;

@@ -63,8 +63,7 @@ __device__ inline double block_sum(double v, double* red) {
 // before a barrier.
 __device__ inline double frame_sum_w64(const double* part, int nblk) {
   double a4[4] = {0.0, 0.0, 0.0, 0.0};
-  const int l = threadIdx.x;
-  int i = l;
+  int i = threadIdx.x & 63;
   for (; i + 960 < nblk; i += 1024) {  // 16 loads in flight, the same order
     double v[16];
 #pragma unroll
@@ -574,10 +573,12 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
 // needs the frame's sum of alpha after the death test, so the pack keeps
 // digamma(alpha) and the E-step subtracts digamma(sum); E[ln det] and
 // E[ln pi] reach the Gaussian's record when that iteration's M-step runs,
-// as the reference computes them at the start of each iteration.
+// as the reference computes them at the start of each iteration. psi:
+// digamma((nu + 1 - i) / 2) for i = 0, 1, 2, then digamma(alpha).
 __device__ inline void gauss_prep_one(const DevPtrs& P, const KOpts& O, const FrameDev* F,
                                       long long k, bool alive, const double* m,
-                                      const double* W, double nu, double beta, double alpha) {
+                                      const double* W, double nu, double beta,
+                                      const double* psi) {
   const long long G = P.Gcap;
   if (!alive) {
     P.eldn[k] = -1e32;
@@ -586,14 +587,14 @@ __device__ inline void gauss_prep_one(const DevPtrs& P, const KOpts& O, const Fr
     return;
   }
   double eld = 3.0 * 0.69314718055994530942 + log(det3(W));
-  for (int i = 0; i < 3; i++) eld += digamma(0.5 * (nu + 1.0 - i));
+  for (int i = 0; i < 3; i++) eld += psi[i];
   P.eldn[k] = eld;
   EPack ep;
   for (int i = 0; i < 3; i++) ep.m[i] = m[i];
   for (int i = 0; i < 6; i++) ep.W[i] = W[i];
   ep.nu = nu;
   ep.kappa0 = 0.5 * eld - 1.5 / beta;
-  ep.dpsi = digamma(alpha);
+  ep.dpsi = psi[3];
   P.epack[k] = ep;
   const float4 mf = make_float4((float)m[0], (float)m[1], (float)m[2], __int_as_float((int)k));
   P.m4[k] = mf;
@@ -619,8 +620,11 @@ __global__ __launch_bounds__(kGB) void k_gauss_prep(DevPtrs P, KOpts O) {
   double m[3], W[6];
   for (int i = 0; i < 3; i++) m[i] = gsv(P, GS_M + i, k);
   for (int i = 0; i < 6; i++) W[i] = gsv(P, GS_W + i, k);
-  gauss_prep_one(P, O, F, k, gsv(P, GS_M_O, k) > -1e31, m, W, gsv(P, GS_NU, k),
-                 gsv(P, GS_BETA, k), gsv(P, GS_ALPHA, k));
+  const double nu = gsv(P, GS_NU, k);
+  double psi[4];
+  for (int i = 0; i < 3; i++) psi[i] = digamma(0.5 * (nu + 1.0 - i));
+  psi[3] = digamma(gsv(P, GS_ALPHA, k));
+  gauss_prep_one(P, O, F, k, gsv(P, GS_M_O, k) > -1e31, m, W, nu, gsv(P, GS_BETA, k), psi);
 }
 
 // Counting-sort scatter of the means into their grid cells; every mean of an
@@ -2058,81 +2062,91 @@ __global__ __launch_bounds__(256) void k_seg_sort(DevPtrs P, int nshort, int nlo
     seg_sort_long(P, sh, (int)blockIdx.x - nshort, nlong);
 }
 
+// Gaussian k after an iteration's posterior update.
+struct GaussState {
+  double m[3], W[6], nu, beta, alpha;
+  double eld;  // E[ln det] of the iteration just run
+  bool alive, fixed;
+};
+
+// nu and alpha of Gaussian k after the posterior update (GMEM.cu:1601-1677),
+// from the M-step's N: changed only when it is alive and not fixed.
+__device__ inline double nu_after(const DevPtrs& P, long long k, bool live, double N) {
+  return live ? gsv(P, GS_NU_O, k) + N : gsv(P, GS_NU, k);
+}
+__device__ inline double alpha_after(const DevPtrs& P, long long k, bool live, double N) {
+  return live ? fmax(gsv(P, GS_ALPHA_O, k) + N, 0.0) : gsv(P, GS_ALPHA, k);
+}
+
 // Posterior (GMEM.cu:1601-1677) and regularisation (GMEM.cu:1693-1809) of
-// Gaussian k from its M-step sums st = (N, S1[3], S2[6]), for an alive,
-// non-fixed Gaussian; commits this iteration's E[ln det] and E[ln pi].
-// Returns alpha_k after the update. Not inlined: one compiled body for every
-// M-step launch shape, so that every shape rounds identically (contraction
-// into fused multiply-adds is decided per compiled body).
-__device__ __noinline__ double mstep_update_one(double* __restrict__ gs,
-                                                const double* __restrict__ eldn,
-                                                const EPack* __restrict__ epack,
-                                                const unsigned char* __restrict__ fixed_flags,
-                                                long long G, long long k, double psi_sum,
-                                                const double* st, int w4dof, float sr0,
-                                                float sr1, float sr2, double lmin, double lmax,
-                                                double emax) {
-#define GSV(fidx, kk) gs[(long long)(fidx) * G + (kk)]
-  const bool alive = GSV(GS_M_O, k) > -1e31;
-  const bool fixed = fixed_flags[k] != 0;
+// Gaussian k from its M-step sums (mst), if it is alive and not fixed;
+// commits this iteration's E[ln det] and E[ln pi].
+__device__ inline GaussState posterior_one(const DevPtrs& P, const KOpts& O, long long k,
+                                           double psi_sum) {
+  const long long G = P.Gcap;
+  double* gs = P.gs;
+  GaussState g;
+  g.alive = gsv(P, GS_M_O, k) > -1e31;
+  g.fixed = P.fixed[k] != 0;
   // this iteration's expectations, as used by its E-step
-  gs[GS_ELD * G + k] = eldn[k];
-  gs[GS_ELP * G + k] = alive ? epack[k].dpsi - psi_sum : -1e32;
-  if (alive && !fixed) {
-    const double r0 = GSV(GS_M, k), r1 = GSV(GS_M + 1, k), r2 = GSV(GS_M + 2, k);
-    const double N = st[0];
-    double S1[3], S2[6];
-    for (int i = 0; i < 3; i++) S1[i] = st[1 + i];
-    for (int i = 0; i < 6; i++) S2[i] = st[4 + i];
-    double xk[3] = {0, 0, 0}, Ck[6] = {0, 0, 0, 0, 0, 0};
-    if (N > 0.0) {
-      const double m0 = S1[0] / N, m1 = S1[1] / N, m2 = S1[2] / N;
-      xk[0] = r0 + m0;
-      xk[1] = r1 + m1;
-      xk[2] = r2 + m2;
-      Ck[0] = S2[0] - S1[0] * m0;
-      Ck[1] = S2[1] - S1[0] * m1;
-      Ck[2] = S2[2] - S1[0] * m2;
-      Ck[3] = S2[3] - S1[1] * m1;
-      Ck[4] = S2[4] - S1[1] * m2;
-      Ck[5] = S2[5] - S1[2] * m2;
-    }
-    // posterior (FP64 throughout)
-    const double beta_o = GSV(GS_BETA_O, k), nu_o = GSV(GS_NU_O, k),
-                 alpha_o = GSV(GS_ALPHA_O, k);
-    double mo[3], Wo[6];
-    for (int i = 0; i < 3; i++) mo[i] = GSV(GS_M_O + i, k);
-    for (int i = 0; i < 6; i++) Wo[i] = GSV(GS_W_O + i, k);
-    const double beta = beta_o + N, nu = nu_o + N, alpha = fmax(alpha_o + N, 0.0);
-    double m[3];
-    for (int i = 0; i < 3; i++) m[i] = (beta_o * mo[i] + N * xk[i]) / beta;
-    if (Wo[5] < 1e-8) {
-      Wo[5] = 0.5 * (Wo[0] + Wo[3]);
-      gs[(GS_W_O + 5) * G + k] = Wo[5];
-    }
-    double A[6], W[6];
-    inv3(Wo, A);
-    const double dx[3] = {xk[0] - mo[0], xk[1] - mo[1], xk[2] - mo[2]};
-    const double fct = beta_o / (beta_o + N);
-    A[0] += Ck[0] + N * fct * dx[0] * dx[0];
-    A[1] += Ck[1] + N * fct * dx[0] * dx[1];
-    A[2] += Ck[2] + N * fct * dx[0] * dx[2];
-    A[3] += Ck[3] + N * fct * dx[1] * dx[1];
-    A[4] += Ck[4] + N * fct * dx[1] * dx[2];
-    A[5] += Ck[5] + N * fct * dx[2] * dx[2];
-    inv3(A, W);
-    const float sreg[3] = {sr0, sr1, sr2};
-    regularize_W(W, nu, w4dof, sreg, lmin, lmax, emax);
-    gs[GS_BETA * G + k] = beta;
-    gs[GS_NU * G + k] = nu;
-    gs[GS_ALPHA * G + k] = alpha;
-    for (int i = 0; i < 3; i++) gs[(GS_M + i) * G + k] = m[i];
-    for (int i = 0; i < 6; i++) gs[(GS_W + i) * G + k] = W[i];
-    return alpha;
-  } else {
-    return GSV(GS_ALPHA, k);
+  g.eld = P.eldn[k];
+  gs[GS_ELD * G + k] = g.eld;
+  gs[GS_ELP * G + k] = g.alive ? P.epack[k].dpsi - psi_sum : -1e32;
+  for (int i = 0; i < 3; i++) g.m[i] = gsv(P, GS_M + i, k);
+  for (int i = 0; i < 6; i++) g.W[i] = gsv(P, GS_W + i, k);
+  const bool live = g.alive && !g.fixed;
+  const double N = P.mst[k];
+  g.nu = nu_after(P, k, live, N);
+  g.alpha = alpha_after(P, k, live, N);
+  if (!live) {
+    g.beta = gsv(P, GS_BETA, k);
+    return g;
   }
-#undef GSV
+  double S1[3], S2[6];
+  for (int i = 0; i < 3; i++) S1[i] = P.mst[(1 + i) * G + k];
+  for (int i = 0; i < 6; i++) S2[i] = P.mst[(4 + i) * G + k];
+  double xk[3] = {0, 0, 0}, Ck[6] = {0, 0, 0, 0, 0, 0};
+  if (N > 0.0) {
+    const double m0 = S1[0] / N, m1 = S1[1] / N, m2 = S1[2] / N;
+    xk[0] = g.m[0] + m0;
+    xk[1] = g.m[1] + m1;
+    xk[2] = g.m[2] + m2;
+    Ck[0] = S2[0] - S1[0] * m0;
+    Ck[1] = S2[1] - S1[0] * m1;
+    Ck[2] = S2[2] - S1[0] * m2;
+    Ck[3] = S2[3] - S1[1] * m1;
+    Ck[4] = S2[4] - S1[1] * m2;
+    Ck[5] = S2[5] - S1[2] * m2;
+  }
+  // posterior (FP64 throughout)
+  const double beta_o = gsv(P, GS_BETA_O, k);
+  double mo[3], Wo[6];
+  for (int i = 0; i < 3; i++) mo[i] = gsv(P, GS_M_O + i, k);
+  for (int i = 0; i < 6; i++) Wo[i] = gsv(P, GS_W_O + i, k);
+  g.beta = beta_o + N;
+  for (int i = 0; i < 3; i++) g.m[i] = (beta_o * mo[i] + N * xk[i]) / g.beta;
+  if (Wo[5] < 1e-8) {
+    Wo[5] = 0.5 * (Wo[0] + Wo[3]);
+    gs[(GS_W_O + 5) * G + k] = Wo[5];
+  }
+  double A[6];
+  inv3(Wo, A);
+  const double dx[3] = {xk[0] - mo[0], xk[1] - mo[1], xk[2] - mo[2]};
+  const double fct = beta_o / (beta_o + N);
+  A[0] += Ck[0] + N * fct * dx[0] * dx[0];
+  A[1] += Ck[1] + N * fct * dx[0] * dx[1];
+  A[2] += Ck[2] + N * fct * dx[0] * dx[2];
+  A[3] += Ck[3] + N * fct * dx[1] * dx[1];
+  A[4] += Ck[4] + N * fct * dx[1] * dx[2];
+  A[5] += Ck[5] + N * fct * dx[2] * dx[2];
+  inv3(A, g.W);
+  regularize_W(g.W, g.nu, O.w4dof, O.scale_reg, O.lmin, O.lmax, O.emax);
+  gs[GS_BETA * G + k] = g.beta;
+  gs[GS_NU * G + k] = g.nu;
+  gs[GS_ALPHA * G + k] = g.alpha;
+  for (int i = 0; i < 3; i++) gs[(GS_M + i) * G + k] = g.m[i];
+  for (int i = 0; i < 6; i++) gs[(GS_W + i) * G + k] = g.W[i];
+  return g;
 }
 
 // One pair's terms added to the M-step sums c (N, S1[3], S2[6]) about the
@@ -2167,15 +2181,19 @@ __device__ inline void mstep_add(double* c, bool use, double rr, double2 m01, do
 //   S2  = sum r [C_s + W_s (mu_s - m_k)(mu_s - m_k)^T]
 // so xbar = m_k + S1/N and sum w (x - xbar)(x - xbar)^T = S2 - S1 S1^T / N,
 // identical to the reference's per-voxel sums over r_sk * img_v
-// (GMEM.cu:1338-1453); then, in the same block, the posterior
-// (GMEM.cu:1601-1677) and regularisation (GMEM.cu:1693-1809) of the alive,
-// non-fixed Gaussians, and the per-64-Gaussian sums of alpha for the death
-// test. A block covers 64 Gaussians with ML lanes each; their sums go
-// through LDS to wave 0, one lane per Gaussian for the update.
+// (GMEM.cu:1338-1453), and the per-64-Gaussian sums of the alpha that the
+// posterior update will give (GMEM.cu:1601-1677; k_death applies it). A block
+// covers 64 Gaussians with ML lanes each.
 // Summation order, identical for every ML: sorted pair e of a Gaussian is
 // added, in increasing e, to class sum e mod 16, and the class sums are
 // combined as ((c + c^8) + ...^4) ...^1.
-template <int ML>
+// The posterior update is not done here: its FP64 chain on one wave of the
+// block kept the other waves' places empty (51 -> 26 us at 60,000 Gaussians
+// with 16 lanes, 109 -> 45 us on 32 uneven frames of 153,000 Gaussians). What
+// is left is the latency of the pair -> moments gathers. VOX: a voxel's
+// moments are 1, its coordinates and zeros, so 12 bytes are read, not 80, and
+// eight pairs a lane are in flight (voxel frame of 4.9M voxels: 166 -> 45 us).
+template <int ML, bool VOX>
 __global__ __launch_bounds__(64 * ML) void k_mstep(DevPtrs P, KOpts O) {
   constexpr int NC = 16 / ML;
   __shared__ double sums[10][64];
@@ -2198,56 +2216,92 @@ __global__ __launch_bounds__(64 * ML) void k_mstep(DevPtrs P, KOpts O) {
     if (mine) {
       const double r0 = gsv(P, GS_M, k), r1 = gsv(P, GS_M + 1, k), r2 = gsv(P, GS_M + 2, k);
       const int st = P.seg_start[k], en = P.seg_start[k + 1];
-      for (int e0 = st; e0 < en; e0 += 16) {
-        if constexpr (NC == 4) {
-          // four entries per lane: one at a time, an entry past the list or
-          // of zero weight skipped (its loads are not issued)
+      if constexpr (VOX) {
+        constexpr int U = 8 / NC;  // rounds of 16 entries whose loads are issued together
+        for (int e0 = st; e0 < en; e0 += 16 * U) {
+          int code[U][NC];
 #pragma unroll
-          for (int q = 0; q < NC; q++) {
-            const int e = e0 + lane + ML * q;
-            if (e >= en) continue;
-            const int code = P.pairs_sorted[e];
-            const long long s = code >> kPairShift;
-            const int j = code & ((1 << kPairShift) - 1);
-            const double r = (double)P.rnk[(long long)j * S + s];
-            const double2* wm = reinterpret_cast<const double2*>(P.wmom + s * 10);
-            const double2 m01 = wm[0], m23 = wm[1], m45 = wm[2], m67 = wm[3], m89 = wm[4];
-            if (!(m01.x != 0.0)) continue;
-            mstep_add(a[q], true, r, m01, m23, m45, m67, m89, r0, r1, r2);
-          }
-        } else {
-          // one or two entries per lane: the entries' loads first (an entry
-          // past the list reads the list's last pair, in range since
-          // e0 < en), then their sums, where an entry past the list or of
-          // zero weight adds exact zeros (its w and r are 0 and its moments
-          // finite): no branch, so no load waits for the previous entry's
-          int code[NC];
+          for (int u = 0; u < U; u++)
 #pragma unroll
-          for (int q = 0; q < NC; q++) {
-            const int e = e0 + lane + ML * q;
-            code[q] = P.pairs_sorted[e < en ? e : en - 1];
-          }
-          float rq[NC];
-          double2 m01[NC], m23[NC], m45[NC], m67[NC], m89[NC];
+            for (int q = 0; q < NC; q++) {
+              const int e = e0 + 16 * u + lane + ML * q;
+              code[u][q] = P.pairs_sorted[e < en ? e : en - 1];
+            }
+          float rq[U][NC], x[U][NC], y[U][NC], z[U][NC];
 #pragma unroll
-          for (int q = 0; q < NC; q++) {
-            const long long s = code[q] >> kPairShift;
-            const int j = code[q] & ((1 << kPairShift) - 1);
-            rq[q] = P.rnk[(long long)j * S + s];
-            // the supervoxel's 10 weighted moments, contiguous (80 bytes)
-            const double2* wm = reinterpret_cast<const double2*>(P.wmom + s * 10);
-            m01[q] = wm[0];
-            m23[q] = wm[1];
-            m45[q] = wm[2];
-            m67[q] = wm[3];
-            m89[q] = wm[4];
-          }
+          for (int u = 0; u < U; u++)
 #pragma unroll
-          for (int q = 0; q < NC; q++) {
-            const int e = e0 + lane + ML * q;
-            const bool use = e < en && m01[q].x != 0.0;
-            mstep_add(a[q], use, (double)rq[q], m01[q], m23[q], m45[q], m67[q], m89[q], r0, r1,
-                      r2);
+            for (int q = 0; q < NC; q++) {
+              const long long s = code[u][q] >> kPairShift;
+              const int j = code[u][q] & ((1 << kPairShift) - 1);
+              rq[u][q] = P.rnk[(long long)j * S + s];
+              x[u][q] = P.anchor[s];  // the voxel itself
+              y[u][q] = P.anchor[S + s];
+              z[u][q] = P.anchor[2 * S + s];
+            }
+          const double2 zero = make_double2(0.0, 0.0);
+#pragma unroll
+          for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int q = 0; q < NC; q++) {
+              const bool use = e0 + 16 * u + lane + ML * q < en;
+              mstep_add(a[q], use, (double)rq[u][q], make_double2(1.0, (double)x[u][q]),
+                        make_double2((double)y[u][q], (double)z[u][q]), zero, zero, zero, r0, r1,
+                        r2);
+            }
+        }
+      } else {
+        for (int e0 = st; e0 < en; e0 += 16) {
+          if constexpr (NC == 4) {
+            // four entries per lane: one at a time, an entry past the list or
+            // of zero weight skipped (its loads are not issued)
+#pragma unroll
+            for (int q = 0; q < NC; q++) {
+              const int e = e0 + lane + ML * q;
+              if (e >= en) continue;
+              const int code = P.pairs_sorted[e];
+              const long long s = code >> kPairShift;
+              const int j = code & ((1 << kPairShift) - 1);
+              const double r = (double)P.rnk[(long long)j * S + s];
+              const double2* wm = reinterpret_cast<const double2*>(P.wmom + s * 10);
+              const double2 m01 = wm[0], m23 = wm[1], m45 = wm[2], m67 = wm[3], m89 = wm[4];
+              if (!(m01.x != 0.0)) continue;
+              mstep_add(a[q], true, r, m01, m23, m45, m67, m89, r0, r1, r2);
+            }
+          } else {
+            // one or two entries per lane: the entries' loads first (an entry
+            // past the list reads the list's last pair, in range since
+            // e0 < en), then their sums, where an entry past the list or of
+            // zero weight adds exact zeros (its w and r are 0 and its moments
+            // finite): no branch, so no load waits for the previous entry's
+            int code[NC];
+#pragma unroll
+            for (int q = 0; q < NC; q++) {
+              const int e = e0 + lane + ML * q;
+              code[q] = P.pairs_sorted[e < en ? e : en - 1];
+            }
+            float rq[NC];
+            double2 m01[NC], m23[NC], m45[NC], m67[NC], m89[NC];
+#pragma unroll
+            for (int q = 0; q < NC; q++) {
+              const long long s = code[q] >> kPairShift;
+              const int j = code[q] & ((1 << kPairShift) - 1);
+              rq[q] = P.rnk[(long long)j * S + s];
+              // the supervoxel's 10 weighted moments, contiguous (80 bytes)
+              const double2* wm = reinterpret_cast<const double2*>(P.wmom + s * 10);
+              m01[q] = wm[0];
+              m23[q] = wm[1];
+              m45[q] = wm[2];
+              m67[q] = wm[3];
+              m89[q] = wm[4];
+            }
+#pragma unroll
+            for (int q = 0; q < NC; q++) {
+              const int e = e0 + lane + ML * q;
+              const bool use = e < en && m01[q].x != 0.0;
+              mstep_add(a[q], use, (double)rq[q], m01[q], m23[q], m45[q], m67[q], m89[q], r0, r1,
+                        r2);
+            }
           }
         }
       }
@@ -2272,65 +2326,104 @@ __global__ __launch_bounds__(64 * ML) void k_mstep(DevPtrs P, KOpts O) {
   __syncthreads();
   if (threadIdx.x >= 64) return;
   const long long k = (long long)blockIdx.x * 64 + threadIdx.x;
-  double st[10];
 #pragma unroll
-  for (int i = 0; i < 10; i++) st[i] = sums[i][threadIdx.x];
-  double alpha_out = 0.0;
+  for (int i = 0; i < 10; i++) P.mst[i * G + k] = sums[i][threadIdx.x];
+  double alpha = 0.0;
   if (P.g_frame[k] == f)
-    alpha_out = mstep_update_one(P.gs, P.eldn, P.epack, P.fixed, G, k, F->psi_sum_alpha, st,
-                                 O.w4dof, O.scale_reg[0], O.scale_reg[1], O.scale_reg[2], O.lmin,
-                                 O.lmax, O.emax);
-  const double t = block_sum<1>(alpha_out, red);
+    alpha = alpha_after(P, k, gsv(P, GS_M_O, k) > -1e31 && P.fixed[k] == 0,
+                        sums[0][threadIdx.x]);
+  const double t = block_sum<1>(alpha, red);
   if (threadIdx.x == 0) P.part_g2[blockIdx.x] = t;
 }
 
-// Dead-cell rule (GMEM.cu:1813-1843), then the log-likelihood parameters and
-// the per-frame sum of alpha used by the log-likelihood and by the next
-// iteration's E[ln pi]. The log-likelihood parameters are stored in base 2:
-// M = nu W log2(e)/2 and lg2 = (log alpha + log det(nu W)/2 - 1.5 log 2pi) log2(e).
-__global__ __launch_bounds__(kGB) void k_death(DevPtrs P, KOpts O) {
+// The posterior and its regularisation from the M-step's sums, the dead-cell
+// rule (GMEM.cu:1813-1843), then the next iteration's E-step constants and
+// binning, the log-likelihood parameters, and the per-frame sum of alpha used
+// by the log-likelihood and by the next iteration's E[ln pi]. The
+// log-likelihood parameters are stored in base 2: M = nu W log2(e)/2 and lg2 =
+// (log alpha + log det(nu W)/2 - 1.5 log 2pi) log2(e).
+// A block takes 64 Gaussians, a lane each, in four waves: what bounds the
+// kernel is one Gaussian's serial FP64 chain (about 1,500 dependent
+// operations; few waves are in flight), so its independent parts run side by
+// side: wave 0 the posterior and the eigenvalue clamps, waves 1 and 2 the four
+// digammas (they need only nu and alpha), wave 3 the frame's sum of alpha;
+// then wave 0 the E-step constants and wave 1 the Cholesky factor. One wave
+// for all: 12.8 us at 200 Gaussians, 22.9 at 60,000, 46 at 153,000; as here
+// 8.7, 23.0 and 41 (700 bytes a Gaussian: 2.6 TB/s).
+__global__ __launch_bounds__(256) void k_death(DevPtrs P, KOpts O) {
   __shared__ double red[1];
+  __shared__ double psi_s[4][64], W_s[6][64], m_s[3][64], nu_s[64], alpha_s[64];
+  __shared__ double sum_alpha_s;
+  __shared__ int alive_s[64];
   const int f = P.gblk_frame[blockIdx.x];
-  if (f < 0) return;
+  if (f < 0) return;  // uniform over the block
   FrameDev* F = P.fr + f;
   if (!F->active) return;
-  // the frame's sum of alpha after the posterior update, from the blocks'
-  // partials in index order (every block of the frame forms the same value)
-  const double sum_alpha2 = frame_sum_w64(P.part_g2 + F->g0 / kGB, F->nbg);
-  const long long k = (long long)blockIdx.x * kGB + threadIdx.x;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const long long k = (long long)blockIdx.x * kGB + l;
   const long long G = P.Gcap;
-  double alpha_out = 0.0;
-  if (P.g_frame[k] == f) {
-    double W[6];
-    bool nanW = isnan(gsv(P, GS_ELD, k));
-    for (int i = 0; i < 6; i++) {
-      W[i] = gsv(P, GS_W + i, k);
-      nanW |= isnan(W[i]);
+  const bool mine = P.g_frame[k] == f;
+  GaussState g;
+  if (w == 3) {
+    // the frame's sum of alpha after the posterior update, from the blocks'
+    // partials in index order (every block of the frame forms the same value)
+    const double t = frame_sum_w64(P.part_g2 + F->g0 / kGB, F->nbg);
+    if (l == 0) sum_alpha_s = t;
+  } else if (w == 0) {
+    if (mine) g = posterior_one(P, O, k, F->psi_sum_alpha);
+  } else if (mine) {
+    const bool live = gsv(P, GS_M_O, k) > -1e31 && P.fixed[k] == 0;
+    const double N = P.mst[k];
+    const double nu = nu_after(P, k, live, N);
+    if (w == 1) {
+      psi_s[0][l] = digamma(0.5 * (nu + 1.0 - 0));
+      psi_s[1][l] = digamma(0.5 * (nu + 1.0 - 1));
+    } else {
+      psi_s[2][l] = digamma(0.5 * (nu + 1.0 - 2));
+      psi_s[3][l] = digamma(alpha_after(P, k, live, N));
     }
-    double alpha = gsv(P, GS_ALPHA, k);
-    bool alive = gsv(P, GS_M_O, k) > -1e31;
-    const bool fixed = P.fixed[k] != 0;
-    if (nanW || (alpha / sum_alpha2 < 1e-5 && alive && !fixed)) {
-      alpha = 0.0;
+  }
+  __syncthreads();
+  if (w == 0 && mine) {
+    bool nanW = isnan(g.eld);
+    for (int i = 0; i < 6; i++) nanW |= isnan(g.W[i]);
+    if (nanW || (g.alpha / sum_alpha_s < 1e-5 && g.alive && !g.fixed)) {
+      g.alpha = 0.0;
       P.gs[GS_ALPHA * G + k] = 0.0;
       for (int i = 0; i < 3; i++) {
         P.gs[(GS_M_O + i) * G + k] = -1e32;
         P.gs[(GS_M + i) * G + k] = -1e32;
+        g.m[i] = -1e32;
       }
       const double I6[6] = {1, 0, 0, 1, 0, 1};
       for (int i = 0; i < 6; i++) {
-        W[i] = I6[i];
+        g.W[i] = I6[i];
         P.gs[(GS_W + i) * G + k] = I6[i];
       }
-      alive = false;
+      g.alive = false;
     }
+    for (int i = 0; i < 6; i++) W_s[i][l] = g.W[i];
+    for (int i = 0; i < 3; i++) m_s[i][l] = g.m[i];
+    nu_s[l] = g.nu;
+    alpha_s[l] = g.alpha;
+    alive_s[l] = g.alive ? 1 : 0;
+  }
+  __syncthreads();
+  if (w == 0) {
+    if (mine) {
+      const double psi[4] = {psi_s[0][l], psi_s[1][l], psi_s[2][l], psi_s[3][l]};
+      gauss_prep_one(P, O, F, k, g.alive, g.m, g.W, g.nu, g.beta, psi);
+    }
+    const double t = block_sum<1>(mine ? g.alpha : 0.0, red);
+    if (l == 0) P.part_g[blockIdx.x] = t;
+  } else if (w == 1 && mine) {
     const double LOG2E = 1.4426950408889634074;
-    const double nu = gsv(P, GS_NU, k);
-    double m[3];
-    for (int i = 0; i < 3; i++) m[i] = gsv(P, GS_M + i, k);
-    gauss_prep_one(P, O, F, k, alive, m, W, nu, gsv(P, GS_BETA, k), alpha);
+    double W[6];
+    for (int i = 0; i < 6; i++) W[i] = W_s[i][l];
+    const double nu = nu_s[l], alpha = alpha_s[l];
+    const bool alive = alive_s[l] != 0;
     LLPack lp;
-    for (int i = 0; i < 3; i++) lp.m[i] = m[i];
+    for (int i = 0; i < 3; i++) lp.m[i] = m_s[i][l];
     // Cholesky factor (FP64) of M = nu W log2(e)/2; a precision matrix that
     // is not positive definite has no density, its terms are dropped
     double M[6];
@@ -2358,10 +2451,7 @@ __global__ __launch_bounds__(kGB) void k_death(DevPtrs P, KOpts O) {
                  ? (log(alpha) + 0.5 * log(dt) - 1.5 * 1.8378770664093454836) * LOG2E
                  : -INFINITY;
     P.llpack[k] = lp;
-    alpha_out = alpha;
   }
-  const double t = block_sum<1>(alpha_out, red);
-  if (threadIdx.x == 0) P.part_g[blockIdx.x] = t;
 }
 
 // A frame's sum of alpha from the Gaussian-block partials of the kernel
@@ -2979,14 +3069,15 @@ static void launch_loglik(const DevPtrs& P, const KOpts& O, hipStream_t st,
 #undef TGMM_LL
 }
 
+template <bool VOX>
 static void launch_mstep(const DevPtrs& P, const KOpts& O, hipStream_t st) {
   const unsigned g = nb(P.Gext, 64);
   if (O.tiles.ms_lanes == 4)
-    k_mstep<4><<<g, 256, 0, st>>>(P, O);
+    k_mstep<4, VOX><<<g, 256, 0, st>>>(P, O);
   else if (O.tiles.ms_lanes == 8)
-    k_mstep<8><<<g, 512, 0, st>>>(P, O);
+    k_mstep<8, VOX><<<g, 512, 0, st>>>(P, O);
   else
-    k_mstep<16><<<g, 1024, 0, st>>>(P, O);
+    k_mstep<16, VOX><<<g, 1024, 0, st>>>(P, O);
 }
 
 template <int KM>
@@ -3066,9 +3157,12 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
   const int nlong = sort_long_blocks(P);
   k_seg_sort<<<nb(P.Gext, 16) + nlong, 256, 0, st>>>(P, (int)nb(P.Gext, 16), nlong);
   if (tk == TK_MSTEP && e0) (void)hipEventRecord(e0, st);
-  launch_mstep(P, O, st);
+  if (O.voxel)
+    launch_mstep<true>(P, O, st);
+  else
+    launch_mstep<false>(P, O, st);
   if (tk == TK_MSTEP && e1) (void)hipEventRecord(e1, st);
-  k_death<<<gb, kGB, 0, st>>>(P, O);
+  k_death<<<gb, 256, 0, st>>>(P, O);
   k_alpha_sum<<<P.nframes, 64, 0, st>>>(P, 1);
   if (tk == TK_LOGLIK && e0) (void)hipEventRecord(e0, st);
   launch_loglik<KM>(P, O, st, tk == TK_LOGLIK ? e1 : nullptr);

@@ -128,6 +128,7 @@ int ws_alloc(Workspace* w, const WsShape& sh, int K) {
   AL(P.svkeep, 17 * G);
   AL(P.part_g, G / kGB);
   AL(P.part_g2, G / kGB);
+  AL(P.mst, 10 * G);
   AL(P.part_s, S / kLLminB);
   AL(P.part_sg, S / 256);
   AL(P.fr, F);
@@ -146,7 +147,7 @@ long long ws_bytes_estimate(const WsShape& sh, int K) {
   const long long S = sh.Scap, G = sh.Gcap, C = sh.Ccap, V = sh.Vcap;
   return 24 * V + S * (16 + 8 + 4 + 12 + 80 + 80 + 12 + 16 + 17LL * K + 1 + 4 + 8) +
          G * (4 + 8 * GS_NFIELDS * 2 + 1 + 96 + 8 + 64 + 12 + 4 + 8 + 12 + 4 + 1 + 16 + 288 +
-              68 + 4 + 4) +
+              68 + 4 + 4 + 80) +
          8 * C + 64 * sh.Fcap;
 }
 
