@@ -77,3 +77,31 @@ def test_fewer_references_than_slots_and_edges():
     assert gd is None and np.array_equal(gi, O.sv_knn(q, r, 2, SCALE)[0])
     with pytest.raises(em.TgmmError):
         em.knnCUDA_(q, r, 12, SCALE)
+
+
+@pytest.mark.parametrize("Q,R", [(1, 1), (15, 63), (16, 64), (17, 65), (63, 257), (65, 4095),
+                                 (129, 4161)])
+@pytest.mark.parametrize("K", [1, 2, 11])
+def test_tile_edges_and_ties_at_the_last_place(Q, R, K):
+    """Partial groups of queries, partial and empty blocks of references, and
+    coordinates on a coarse lattice (ties among the largest slots, equal
+    centroids) with a flat axis."""
+    rng = np.random.default_rng(Q * 1000 + R + K)
+    print("svknn Q=%d R=%d K=%d" % (Q, R, K), flush=True)
+    for top in (4, 60):
+        q = rng.integers(0, top, (3, Q)).astype(np.float32)
+        r = rng.integers(0, top, (3, R)).astype(np.float32)
+        q[2] = r[2] = 7.0
+        r = r[:, np.lexsort((r[0], r[1], r[2]))]
+        _check(q.reshape(-1), np.ascontiguousarray(r).reshape(-1), K)
+    _check(q.reshape(-1), np.ascontiguousarray(r[:, ::-1]).reshape(-1), K, scale=(1.0, 0.5, 3.0))
+
+
+def test_coordinates_beyond_the_filter_take_every_reference():
+    rng = np.random.default_rng(8)
+    q = rng.uniform(-20, 20, (3, 90)).astype(np.float32)
+    r = rng.uniform(-20, 20, (3, 200)).astype(np.float32)
+    q[0, 5], q[1, 6], r[2, 7], r[0, 100] = np.inf, 3e18, -np.inf, np.nan
+    _check(q.reshape(-1), r.reshape(-1), 7)
+    _check(rng.uniform(0, 9, (3, 40)).astype(np.float32).reshape(-1),
+           rng.uniform(0, 9, (3, 130)).astype(np.float32).reshape(-1), 3, scale=(0.0, 1.0, 2.0))
