@@ -279,7 +279,8 @@ typedef struct tgmm_batch_stats_t {
 int tgmm_batch_stats(tgmm_batch* b, tgmm_batch_stats_t* stats);
 /* Launch shapes of the tunable kernels. Every valid choice gives bitwise the
  * same results (the kernels fix their summation order independently of the
- * shape); only the speed changes. Defaults: {16, 4, 16, 256, 256, 8, 6, 2}. */
+ * shape); only the speed changes. Until set or tuned they are chosen from the
+ * numbers of supervoxels and Gaussians, around {16, 4, 16, 256, 256, 8, 6, 2}. */
 typedef struct tgmm_tiles {
   int ll_group;    /* log-likelihood: 16 or 32 for 2 * ll_group supervoxels
                       per block of 256 threads (32 for K > 8), 64 for 16
@@ -295,7 +296,8 @@ typedef struct tgmm_tiles {
   int knn_cell;    /* mean Gaussians per kNN grid cell: 2, 4 or 6 */
   int knn_lanes;   /* kNN search: 0 = one block of knn_block/64 waves per grid
                       cell, its 3x3x3 block staged in LDS for all of the
-                      cell's queries; 1, 2 or 4 = lanes per query */
+                      cell's queries; 1, 2 or 4 = lanes per query; 64 = a wave
+                      per query (small batches) */
 } tgmm_tiles;
 
 /* A change of knn_cell rebuilds the kNN grids and resets the batch to its

@@ -27,6 +27,7 @@ constexpr int kCB = 64;          // grid-cell range alignment (cell block -> fra
 constexpr int kSB = 256;         // threads per block, supervoxel-lane kernels
 constexpr int kLLminB = 4;       // fewest supervoxels per log-likelihood block
 constexpr int kPairShift = 4;    // pair code = (s << 4) | j, j < 16
+constexpr int kMovedCap = 4;     // moved positions kept per kNN grid cell
 
 // state field indices (record order, GMEMupdateCUDA.h:22-34)
 enum {
@@ -52,6 +53,7 @@ struct FrameDev {
   int iter;           // reference numIterEM (starts at 1)
   int active;         // keeps iterating
   int status;
+  int moved;          // means that moved since the last kNN search
   int packed;         // every voxel's offset from its supervoxel's anchor is a
                       // small integer: the log-likelihood reads vpk (set to 1
                       // on the host, cleared by the moments kernel)
@@ -93,10 +95,13 @@ struct Tiles {
                   // when its grid is built)
   int knn_lanes;  // kNN search: 0 = one block of knn_block/64 waves per grid
                   // cell (its 3x3x3 block staged in LDS for all of the cell's
-                  // queries); 1, 2, 4 = lanes per query
+                  // queries); 1, 2, 4 = lanes per query; 64 = a wave per query
 };
 constexpr Tiles kDefaultTiles = {16, 4, 16, 256, 256, 8, 6, 2};
 bool tiles_valid(const Tiles& t);
+// The launch shapes for S supervoxels and G Gaussians (all frames together)
+// when the caller sets none.
+Tiles tiles_for(long long S, long long G, int K, bool voxel);
 
 struct KOpts {
   int K;
@@ -131,7 +136,7 @@ struct DevPtrs {
   int* sblk_frame;  // Scap/256
   float4* q4;       // Scap: kNN queries of each frame in grid-cell order:
                     // centroid x, y, z and the supervoxel index (int bits)
-  int* qcell;       // Scap: grid cell of each supervoxel centroid
+  int* qcell;       // Scap: grid cell of each kNN query, in q4's order
   // Gaussians
   int* g_frame;
   double* gs;       // 27*Gcap
@@ -159,21 +164,29 @@ struct DevPtrs {
   int* qcell_start; // Ccap+1: first kNN query of each cell (positions in q4)
   int* cblk_frame;  // Ccap/kCB: frame of each 64-cell block, -1 if none
   float4* cg4;      // Gcap: cell-sorted references (x, y, z, index bits)
+  int* cell_mv;     // Ccap+1: old and new positions in the cell of means that moved
+                    // since the last kNN search
+  float4* mv_pos;   // kMovedCap*Ccap: the first of them
   // kNN: supervoxels whose K-th distance is tied with a Gaussian outside
   // their K best (their candidate set follows the reference's scan order)
-  int* tie_list;    // Scap
+  int* tie_list;    // Scap (while a frame is set up: the queries' grid cells)
   int* knn_ctl;     // [0] ties listed this iteration, [1] supervoxels whose
                     //     final slot layout found a different set (stays 0),
-                    //     [2] Gaussians in long_list this iteration
+                    //     [2] Gaussians in long_list this iteration,
+                    //     [3] queries to search for again this iteration (listed
+                    //     in pairs), [4] ties among them
   int* long_list;   // Gcap: Gaussians whose pair list is long (sorted by a block each)
-  int2* win;        // Scap: (Gaussian, slot) of the candidate with r > 0.5, or -1
+  int2* win;        // Scap, after a solve: (Gaussian, slot) of the candidate with
+                    // r > 0.5, or -1; while it runs, in q4's order: what each
+                    // query's last search left (a float, knn_left)
   // results
-  GaussianMixtureModelCUDA* rec;  // Gcap: records as returned (288 B each)
+  GaussianMixtureModelCUDA* rec;  // Gcap: records as returned (288 B each); while
+                                  // a frame iterates, the M-step's sums N, S1[3],
+                                  // S2[6] at the start of each Gaussian's
   int* svkeep;      // 17*Gcap: supervoxelIdx[16] and supervoxelNum as given
   // reductions
   double* part_g;   // Gcap/kGB
   double* part_g2;  // Gcap/kGB: sums of alpha after the posterior update (death test)
-  double* mst;      // 10*Gcap: the M-step's sums N, S1[3], S2[6], field-major
   double* part_s;   // Scap/kLLminB: log-likelihood block partials
   double* part_sg;  // Scap/256: partials of 256-supervoxel groups
   FrameDev* fr;

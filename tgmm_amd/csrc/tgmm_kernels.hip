@@ -80,6 +80,10 @@ __device__ inline double frame_sum_w64(const double* part, int nblk) {
 }
 
 __device__ inline double gsv(const DevPtrs& P, int f, long long k) { return P.gs[f * P.Gcap + k]; }
+// the M-step's sums of Gaussian k (10 doubles, 16-byte aligned)
+__device__ inline double2* msums(const DevPtrs& P, long long k) {
+  return reinterpret_cast<double2*>(P.rec + k);
+}
 
 // reference loop condition (GMEM.cu:4145-4148)
 __device__ inline int keep_going(double ll, double l1, double l2, double l3, double tol) {
@@ -112,6 +116,13 @@ __device__ inline int axis_cell(double u, float org, float h, int dim) {
   if (t >= (double)dim) return dim - 1;
   if (t > 0.0) return (int)floor(t);
   return 0;
+}
+
+// Orders of the LDS accesses of one wave's lanes (no block barrier).
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // ------------------------------------------------------------ prep kernels --
@@ -372,7 +383,7 @@ __global__ __launch_bounds__(256) void k_qcell_count(DevPtrs P, KOpts O) {
     c[a] = axis_cell((double)P.sv_cent[a * S + s] * (double)O.scale[a], F->org[a], F->h,
                      F->dims[a]);
   const long long cell = F->c0 + ((long long)c[2] * F->dims[1] + c[1]) * F->dims[0] + c[0];
-  P.qcell[s] = (int)cell;
+  P.tie_list[s] = (int)cell;
   atomicAdd(P.cell_cnt + cell, 1);
 }
 
@@ -382,10 +393,10 @@ __global__ __launch_bounds__(256) void k_qcell_scatter(DevPtrs P) {
   if (f < 0 || (P.only_frame >= 0 && f != P.only_frame)) return;
   const long long s = sb * 256 + threadIdx.x;
   if (P.sv_frame[s] != f) return;
-  const FrameDev* F = P.fr + f;
-  const int c = P.qcell[s];
+  const int c = P.tie_list[s];
   const long long pos = P.qcell_start[c] + atomicSub(P.cell_cnt + c, 1) - 1;
   const long long S = P.Scap;
+  P.qcell[pos] = c;
   P.q4[pos] = make_float4(P.sv_cent[s], P.sv_cent[S + s], P.sv_cent[2 * S + s],
                           __int_as_float((int)s));
 }
@@ -455,11 +466,14 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
   if (which == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
     P.knn_ctl[0] = 0;
     P.knn_ctl[2] = 0;  // and the list of long pair lists
+    P.knn_ctl[3] = 0;  // and the queries to search for again
+    P.knn_ctl[4] = 0;
   }
   const int f = (P.only_frame >= 0) ? P.only_frame : (int)blockIdx.x;
   if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
   const FrameDev* F = P.fr + f;
   if (F->ncap == 0 || (need_active && !F->active)) return;  // empty slot / finished
+  if (which == 0 && threadIdx.x == 0) P.fr[f].moved = 0;
   const int* in;
   int* out;
   long long n;
@@ -487,6 +501,10 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
 #pragma unroll
     for (int q = 0; q < kScanQ; q++) {
       const long long e = c0 + 4096LL * q + 4LL * threadIdx.x;
+      // the grid scan also clears the moved-mean counts of the frame's cells
+      // (a range has a multiple of 64 entries, more than n)
+      if (which == 0 && e < n)
+        *reinterpret_cast<int4*>(P.cell_mv + F->c0 + e) = make_int4(0, 0, 0, 0);
       if (e + 4 <= n) {
         v[q] = *reinterpret_cast<const int4*>(in + e);
       } else {
@@ -568,6 +586,15 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
 }
 
 // ------------------------------------------------------- iteration kernels --
+// Grid cell (global) of an f32 mean.
+__device__ inline long long mean_cell(const KOpts& O, const FrameDev* F, float4 m) {
+  int c[3];
+  c[0] = axis_cell((double)m.x * (double)O.scale[0], F->org[0], F->h, F->dims[0]);
+  c[1] = axis_cell((double)m.y * (double)O.scale[1], F->org[1], F->h, F->dims[1]);
+  c[2] = axis_cell((double)m.z * (double)O.scale[2], F->org[2], F->h, F->dims[2]);
+  return F->c0 + ((long long)c[2] * F->dims[1] + c[1]) * F->dims[0] + c[0];
+}
+
 // E-step constants and kNN grid binning of Gaussian k for the next iteration
 // (GMEM.cu:553-628, 527-539), from its state (m, W, nu, beta, alpha). E[ln pi]
 // needs the frame's sum of alpha after the death test, so the pack keeps
@@ -598,11 +625,7 @@ __device__ inline void gauss_prep_one(const DevPtrs& P, const KOpts& O, const Fr
   P.epack[k] = ep;
   const float4 mf = make_float4((float)m[0], (float)m[1], (float)m[2], __int_as_float((int)k));
   P.m4[k] = mf;
-  int c[3];
-  c[0] = axis_cell((double)mf.x * (double)O.scale[0], F->org[0], F->h, F->dims[0]);
-  c[1] = axis_cell((double)mf.y * (double)O.scale[1], F->org[1], F->h, F->dims[1]);
-  c[2] = axis_cell((double)mf.z * (double)O.scale[2], F->org[2], F->h, F->dims[2]);
-  const long long cell = F->c0 + ((long long)c[2] * F->dims[1] + c[1]) * F->dims[0] + c[0];
+  const long long cell = mean_cell(O, F, mf);
   P.gcell[k] = (int)cell;
   atomicAdd(P.cell_cnt + cell, 1);
 }
@@ -627,21 +650,38 @@ __global__ __launch_bounds__(kGB) void k_gauss_prep(DevPtrs P, KOpts O) {
   gauss_prep_one(P, O, F, k, gsv(P, GS_M_O, k) > -1e31, m, W, nu, gsv(P, GS_BETA, k), psi);
 }
 
+__device__ inline void list_moved(const DevPtrs& P, long long cell, float4 m) {
+  const int n = atomicAdd(P.cell_mv + cell, 1);
+  if (n < kMovedCap) P.mv_pos[cell * kMovedCap + n] = m;
+}
+
 // Counting-sort scatter of the means into their grid cells; every mean of an
 // active frame (NaN when dead) is also kept in index order as the means of
 // this iteration's kNN search (m4 is rewritten for the next iteration before
-// the search's slot layout is replayed after the last one).
-__global__ __launch_bounds__(kGB) void k_grid_scatter(DevPtrs P) {
+// the search's slot layout is replayed after the last one). A mean that is
+// not bitwise where the last search saw it is listed in its old cell and in
+// its new one (after the first iteration, which searches for every query).
+__global__ __launch_bounds__(kGB) void k_grid_scatter(DevPtrs P, KOpts O) {
   const int f = P.gblk_frame[blockIdx.x];
   if (f < 0 || !P.fr[f].active) return;
+  const FrameDev* F = P.fr + f;
   const long long k = (long long)blockIdx.x * kGB + threadIdx.x;
   if (P.g_frame[k] != f) return;
-  const float4 m = P.m4[k];
+  const float4 m = P.m4[k], old = P.mknn[k];
   P.mknn[k] = m;
   const int c = P.gcell[k];
-  if (c < 0) return;
-  const int pos = P.cell_start[c] + atomicSub(P.cell_cnt + c, 1) - 1;
-  P.cg4[pos] = m;
+  if (c >= 0) {
+    const int pos = P.cell_start[c] + atomicSub(P.cell_cnt + c, 1) - 1;
+    P.cg4[pos] = m;
+  }
+  if (F->iter > 1 && (__float_as_int(m.x) != __float_as_int(old.x) ||
+                      __float_as_int(m.y) != __float_as_int(old.y) ||
+                      __float_as_int(m.z) != __float_as_int(old.z))) {
+    if (c >= 0) list_moved(P, c, m);
+    if (old.x == old.x) list_moved(P, mean_cell(O, F, old), old);  // not dead then
+    const unsigned long long here = __ballot(1);
+    if (__lane_id() == __builtin_ctzll(here)) atomicAdd(&P.fr[f].moved, __popcll(here));
+  }
 }
 
 // Inserts a candidate (distance d <= 1e32, index idx) into a list of the KM
@@ -714,8 +754,9 @@ __device__ inline void knn_merge(float (&bd)[KM], int (&bi)[KM], int K, bool& ti
 // reference that can enter the K best. QL lanes share a query (lane `sub`
 // takes every QL-th reference of a range); their lists are merged after each
 // shell.
+// Returns whether the first block sufficed.
 template <int KM, int QL, typename Consider, typename Flush>
-__device__ inline void knn_shells(const DevPtrs& P, const FrameDev* F, const int* c,
+__device__ inline bool knn_shells(const DevPtrs& P, const FrameDev* F, const int* c,
                                   const double* u, int K, int sub, float (&bd)[KM],
                                   int (&bi)[KM], bool& tie, float& kd, Consider consider,
                                   Flush flush) {
@@ -791,8 +832,9 @@ __device__ inline void knn_shells(const DevPtrs& P, const FrameDev* F, const int
       if (QL > 1) knn_merge<KM, QL>(bd, bi, K, tie, kd);
     }
     const double lb2 = lower_bound_sq(r);
-    if (lb2 == INFINITY || kth() < lb2) break;  // every cell visited, or done
+    if (lb2 == INFINITY || kth() < lb2) return r == 1;  // every cell visited, or done
   }
+  return false;
 }
 
 // Exact K nearest means by expanding shells of grid cells. After shell r,
@@ -810,16 +852,68 @@ __device__ inline void knn_shells(const DevPtrs& P, const FrameDev* F, const int
 // kKnnQueue entries per thread).
 constexpr int kKnnQueue = 20;
 
+// What a search leaves for later iterations (in win, in q4's order): the K-th
+// distance, or -1 when the query is to be searched again whatever moved (its
+// K-th distance was tied, fewer than K means live, or its K nearest reach
+// beyond the 3x3x3 block of its cell).
+__device__ inline float* knn_left(const DevPtrs& P, long long i) {
+  return reinterpret_cast<float*>(P.win + i);
+}
+
+// Whether query i may have other nearest means than at its last search. Its K
+// nearest, and a tie at the K-th distance, can change only through a mean
+// that was or now is within the K-th distance; every such place lies in the
+// 3x3x3 block of cells around its own (whatever lies outside is farther than
+// the K-th distance by the block's bound), so the means that moved are looked
+// up in those cells. A query near a cell with more moved positions than it
+// keeps is searched again.
+// In the EM's later iterations most means do not move at all in f32 (frame of
+// 60,000 Gaussians: 1% move in the 7th iteration, 0.1% in the 12th).
+__device__ inline bool knn_needed(const float* win, const int* qcell, const int* cell_mv,
+                                  const float4* mv_pos, const float4* q4, const FrameDev* F,
+                                  float s0, float s1, float s2, long long i) {
+  const float kd = win[2 * i];
+  const int cell = qcell[i];
+  if (!(kd >= 0.0f)) return true;
+  const int nx = F->dims[0], ny = F->dims[1], nz = F->dims[2];
+  const long long c0 = F->c0;
+  const unsigned c = (unsigned)(cell - c0);
+  const unsigned t = c / (unsigned)nx;
+  const int x = (int)(c - t * nx), z = (int)(t / (unsigned)ny), y = (int)(t - (unsigned)z * ny);
+  // the block's counts in one round of loads (cells past an edge read the
+  // edge's again), then the few cells that hold any
+  unsigned mask = 0u;
+#pragma unroll
+  for (int o = 0; o < 27; o++) {
+    const int zz = min(max(z + o / 9 - 1, 0), nz - 1), yy = min(max(y + o / 3 % 3 - 1, 0), ny - 1),
+              xx = min(max(x + o % 3 - 1, 0), nx - 1);
+    mask |= cell_mv[c0 + (zz * ny + yy) * nx + xx] != 0 ? 1u << o : 0u;
+  }
+  if (mask == 0u) return false;
+  const float4 q = q4[i];
+  while (mask) {
+    const int o = __builtin_ctz(mask);
+    mask &= mask - 1u;
+    const int zz = min(max(z + o / 9 - 1, 0), nz - 1), yy = min(max(y + o / 3 % 3 - 1, 0), ny - 1),
+              xx = min(max(x + o % 3 - 1, 0), nx - 1);
+    const long long at = c0 + (zz * ny + yy) * nx + xx;
+    const int n = cell_mv[at];
+    bool hit = n > kMovedCap;
+#pragma unroll
+    for (int e = 0; e < kMovedCap; e++) {
+      const float4 m = mv_pos[at * kMovedCap + e];
+      hit |= e < n && knn_dist(q.x, q.y, q.z, m.x, m.y, m.z, s0, s1, s2) <= kd;
+    }
+    if (hit) return true;
+  }
+  return false;
+}
+
+// The exact search for query i by its QL lanes (lane sub); kq: the block's
+// candidate queues, entry e of thread t at e * blockDim.x + t.
 template <int KM, int KC, int QL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KM <= 8 ? 4 : 1))) void k_knn(DevPtrs P, KOpts O) {
-  extern __shared__ float2 kq[];  // entry e of thread t at e * blockDim.x + t
-  const int sub = threadIdx.x % QL;
-  const long long qpb = blockDim.x / QL;  // queries per block
-  const long long i = (long long)blockIdx.x * qpb + threadIdx.x / QL;
-  const int f = P.sblk_frame[((long long)blockIdx.x * qpb) >> 8];
-  if (f < 0 || !P.fr[f].active) return;
-  const FrameDev* F = P.fr + f;
-  if (i >= F->s0 + F->ns) return;  // the whole group of the query leaves
+__device__ __forceinline__ void knn_search(const DevPtrs& P, const KOpts& O, const FrameDev* F,
+                                           long long i, int sub, float2* kq) {
   const float4 qq = P.q4[i];
   const long long s = __float_as_int(qq.w);
   const long long S = P.Scap;
@@ -974,15 +1068,241 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KM <= 8 ? 4
       }
     }
   };
-  knn_shells<KM, QL>(P, F, c, u, K, sub, bd, bi, tie, kd, defer, flush);
+  const bool block = knn_shells<KM, QL>(P, F, c, u, K, sub, bd, bi, tie, kd, defer, flush);
 #pragma unroll
   for (int m = QL / 2; m >= 1; m >>= 1) tie |= __shfl_xor((int)tie, m, QL) != 0;
   if (sub == 0) {
 #pragma unroll
     for (int j = 0; j < KM; j++)
       if (j < K) P.ind[(long long)j * S + s] = (bd[j] <= 1e32f) ? bi[j] : -1;
+    // kd is infinite while fewer than K are held
+    *knn_left(P, i) = block && !tie && kd <= 1e32f ? kd : -1.0f;
     if (tie) P.tie_list[atomicAdd(P.knn_ctl, 1)] = (int)s;
   }
+}
+
+// The same search by a whole wave for one query: a lane a reference, the K
+// best spread over the first K lanes in (distance, index) order. Every row of
+// cells of a shell is looked up at once and its references follow 256 at a
+// time, so a query takes a few rounds of loads however many shells it needs
+// (the lane search above goes row by row; its latency is about 14 us). lds:
+// 256 ints of this wave's own. Returns whether the K-th distance is tied.
+template <int KM>
+__device__ inline bool knn_wave(const DevPtrs& P, const KOpts& O, const FrameDev* F, long long i,
+                                int* lds) {
+  const int lane = threadIdx.x & 63;
+  const int K = O.K;
+  const long long S = P.Scap;
+  const float s0 = O.scale[0], s1 = O.scale[1], s2 = O.scale[2];
+  const int nx = F->dims[0], ny = F->dims[1], nz = F->dims[2];
+  const int dims[3] = {nx, ny, nz};
+  const double h = F->h;
+  const double org[3] = {F->org[0], F->org[1], F->org[2]};
+  const float4 qq = P.q4[i];
+  const long long s = __float_as_int(qq.w);
+  const float q0 = qq.x, q1 = qq.y, q2 = qq.z;
+  const double u[3] = {(double)q0 * s0, (double)q1 * s1, (double)q2 * s2};
+  int c[3];
+  {
+    const int cell = (int)(P.qcell[i] - F->c0), t = cell / nx;
+    c[0] = cell - t * nx;
+    c[2] = t / ny;
+    c[1] = t - c[2] * ny;
+  }
+  // the bound of the K-th distance, as in knn_search
+  float kbound = INFINITY;
+  {
+    const int k = lane < K ? P.ind[(long long)lane * S + s] : -1;
+    const bool in = k >= F->g0 && k < F->g0 + F->ng;
+    const float4 m = P.m4[in ? k : 0];
+    const float d = in ? knn_dist(q0, q1, q2, m.x, m.y, m.z, s0, s1, s2) : NAN;
+    const bool ok = d <= 1e32f;
+    float mx = lane < K ? d : -INFINITY;
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if (__ballot(lane < K && !ok) == 0ull) kbound = __shfl(mx, 0, 64);
+  }
+  float ld = INFINITY, kd = INFINITY, out = INFINITY;
+  int li = 0x7fffffff, ki = 0x7fffffff;
+  auto consider = [&](bool have, float4 r) {
+    const float d = have ? knn_dist(q0, q1, q2, r.x, r.y, r.z, s0, s1, s2) : INFINITY;
+    const int idx = __float_as_int(r.w);
+    const bool ok = d <= kbound && d <= 1e32f;
+    const bool better = ok && lex_less(d, idx, kd, ki);
+    if (ok && !better) out = fminf(out, d);
+    unsigned long long m = __ballot(better);
+    while (m) {
+      const int l = __builtin_ctzll(m);
+      m &= m - 1ull;
+      const float cd = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), l));
+      const int ci = __builtin_amdgcn_readlane(idx, l);
+      if (!lex_less(cd, ci, kd, ki)) {
+        out = fminf(out, cd);
+        continue;
+      }
+      out = fminf(out, kd);  // the K-th leaves (infinite while fewer are held)
+      const int rank = __popcll(__ballot(lane < K && lex_less(ld, li, cd, ci)));
+      const float pd = __shfl_up(ld, 1, 64);
+      const int pi = __shfl_up(li, 1, 64);
+      ld = lane > rank ? pd : (lane == rank ? cd : ld);
+      li = lane > rank ? pi : (lane == rank ? ci : li);
+      kd = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ld), K - 1));
+      ki = __builtin_amdgcn_readlane(li, K - 1);
+    }
+  };
+  auto box_d2 = [&](int a, int ci) -> double {
+    const double lo = org[a] + (double)ci * h, hi = org[a] + (double)(ci + 1) * h;
+    const double d = fmax(fmax(lo - u[a], u[a] - hi), 0.0) * (1.0 - 1e-5);
+    return d * d;
+  };
+  int* pre = lds;
+  int* beg0 = lds + 64;
+  int* len0 = lds + 128;
+  int* beg1 = lds + 192;
+  const int rmax = max(nx, max(ny, nz));
+  int reach = 0;
+  for (int r = 1; r <= rmax; r++) {
+    const int w = 2 * r + 1;
+    for (int t0 = 0; t0 < w * w; t0 += 64) {
+      const int t = t0 + lane;
+      const int dz = t / w - r, dy = t - (t / w) * w - r;
+      const int z = c[2] + dz, y = c[1] + dy;
+      int b0 = 0, n0 = 0, b1 = 0, n1 = 0;
+      if (t < w * w && z >= 0 && z < nz && y >= 0 && y < ny &&
+          box_d2(2, z) + box_d2(1, y) <= (double)fminf(kbound, kd)) {
+        const int* cs = P.cell_start + F->c0 + ((long long)z * ny + y) * nx;
+        if (r == 1 || dz == -r || dz == r || dy == -r || dy == r) {
+          b0 = cs[max(c[0] - r, 0)];
+          n0 = cs[min(c[0] + r, nx - 1) + 1] - b0;
+        } else {  // an inner row's two end cells
+          if (c[0] - r >= 0) {
+            b0 = cs[c[0] - r];
+            n0 = cs[c[0] - r + 1] - b0;
+          }
+          if (c[0] + r < nx) {
+            b1 = cs[c[0] + r];
+            n1 = cs[c[0] + r + 1] - b1;
+          }
+        }
+      }
+      int x = n0 + n1;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(x, o, 64);
+        if (lane >= o) x += v;
+      }
+      const int tot = __shfl(x, 63, 64);
+      wave_lds_sync();  // the rows before have been read
+      pre[lane] = x - n0 - n1;
+      beg0[lane] = b0;
+      len0[lane] = n0;
+      beg1[lane] = b1;
+      wave_lds_sync();
+      for (int j0 = 0; j0 < tot; j0 += 256) {
+        float4 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int j = j0 + 64 * q + lane;
+          v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (j < tot) {
+            int lo = 0;  // the last row that starts at or before j
+#pragma unroll
+            for (int st = 32; st >= 1; st >>= 1)
+              if (pre[lo + st] <= j) lo += st;
+            const int o = j - pre[lo];
+            v[q] = P.cg4[o < len0[lo] ? beg0[lo] + o : beg1[lo] + o - len0[lo]];
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (j0 + 64 * q < tot) consider(j0 + 64 * q + lane < tot, v[q]);
+      }
+    }
+    // the open-face bound of the visited block, as in knn_shells
+    double lb = INFINITY;
+    for (int a = 0; a < 3; a++) {
+      if (c[a] - r > 0) lb = fmin(lb, u[a] - (org[a] + (double)(c[a] - r) * h));
+      if (c[a] + r < dims[a] - 1) lb = fmin(lb, (org[a] + (double)(c[a] + r + 1) * h) - u[a]);
+    }
+    if (lb < INFINITY) lb = fmax(lb, 0.0) * (1.0 - 1e-5);
+    if (lb == INFINITY || (double)kd < lb * lb) {
+      reach = r;
+      break;
+    }
+  }
+  const bool tie = __ballot(out == kd && kd <= 1e32f) != 0ull;
+  if (lane < K) P.ind[(long long)lane * S + s] = ld <= 1e32f ? li : -1;
+  if (lane == 0)
+    *knn_left(P, i) = reach == 1 && !tie && kd <= 1e32f ? kd : -1.0f;
+  return tie;
+}
+
+// Whether this iteration only looks for queries whose neighbours may have
+// changed, or searches for every query: the first iteration, and those in
+// which more than 1/128 of the frame's means moved. With a share p moved,
+// about 1 - (1 - p)^2K of the queries have to be searched again; by waves
+// that costs about five times a query of the lane search, so the line lies
+// where some tenth of the queries is left.
+__device__ inline bool knn_looks(const FrameDev* F) {
+  return F->iter > 1 && 128LL * F->moved <= F->ng;
+}
+
+// The look over every query, a lane each: those that may have other neighbours
+// are listed (k_knn_exact searches for them), the others keep the candidates
+// they have. The list lies in the pair runs, which are written later in the
+// iteration. A kernel of its own: beside the lane search in one body it costs
+// that search registers (60,000 Gaussians: 176 -> 215 us).
+__global__ __launch_bounds__(256) void k_knn_look(DevPtrs P, KOpts O) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int f = P.sblk_frame[blockIdx.x];
+  if (f < 0 || !P.fr[f].active) return;
+  const FrameDev* F = P.fr + f;
+  if (!knn_looks(F)) return;
+  const bool need =
+      i < F->s0 + F->ns && knn_needed(knn_left(P, 0), P.qcell, P.cell_mv, P.mv_pos, P.q4, F,
+                                      O.scale[0], O.scale[1], O.scale[2], i);
+  const unsigned long long m = __ballot(need);
+  if (m == 0ull) return;
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (lane == 0) base = atomicAdd(P.knn_ctl + 3, __popcll(m));
+  base = __builtin_amdgcn_readfirstlane(base);
+  if (need) P.pairs[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)i;
+}
+
+// The lane search of every query, blockDim.x / QL a block.
+// VALU-bound: 5.7k instructions a wave at K = 8 (60,000 Gaussians: 152 us).
+template <int KM, int KC, int QL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KM <= 8 ? 4 : 1))) void k_knn(DevPtrs P, KOpts O) {
+  extern __shared__ float2 kq[];
+  const long long qpb = blockDim.x / QL;  // queries per block
+  const long long i = (long long)blockIdx.x * qpb + threadIdx.x / QL;
+  const int f = P.sblk_frame[((long long)blockIdx.x * qpb) >> 8];
+  if (f < 0 || !P.fr[f].active) return;
+  const FrameDev* F = P.fr + f;
+  if (knn_looks(F)) return;
+  if (i >= F->s0 + F->ns) return;  // the whole group of the query leaves
+  knn_search<KM, KC, QL>(P, O, F, i, threadIdx.x % QL, kq);
+}
+
+// A wave per query (knn_lanes 64, for small batches): every query at once,
+// each looked over first. The lane search's latency on 900 queries is 16.5 us,
+// this is 6.2.
+template <int KM>
+__global__ __launch_bounds__(256) void k_knn_small(DevPtrs P, KOpts O) {
+  __shared__ int rows[4][256];
+  const int w = threadIdx.x >> 6;
+  const long long i = (long long)blockIdx.x * 4 + w;
+  const int f = P.sblk_frame[i >> 8];
+  if (f < 0 || !P.fr[f].active) return;
+  const FrameDev* F = P.fr + f;
+  if (i >= F->s0 + F->ns) return;  // whole waves
+  if (F->iter > 1 && !knn_needed(knn_left(P, 0), P.qcell, P.cell_mv, P.mv_pos, P.q4, F, O.scale[0],
+                                 O.scale[1], O.scale[2], i))
+    return;
+  const bool tie = knn_wave<KM>(P, O, F, i, rows[w]);
+  if (tie && (threadIdx.x & 63) == 0)
+    P.tie_list[atomicAdd(P.knn_ctl, 1)] = __float_as_int(P.q4[i].w);
 }
 
 // Exact K nearest means, one block per grid cell (the same search as k_knn,
@@ -1012,6 +1332,7 @@ __global__ __launch_bounds__(64 * NW) void k_knn_cell(DevPtrs P, KOpts O) {
   if (lc >= (long long)nx * ny * nz) return;
   const int qs = P.qcell_start[cc], qe = P.qcell_start[cc + 1];
   if (qs >= qe) return;
+  if (knn_looks(F)) return;
   const long long c0 = F->c0;
   const int c[3] = {(int)(lc % nx), (int)((lc / nx) % ny), (int)(lc / ((long long)nx * ny))};
   // the 9 rows of the block: lanes 0..8 read the row starts, 9..17 the ends
@@ -1103,10 +1424,11 @@ __global__ __launch_bounds__(64 * NW) void k_knn_cell(DevPtrs P, KOpts O) {
     }
     if (!act) continue;
     const double u[3] = {(double)q0 * s0, (double)q1 * s1, (double)q2 * s2};
-    knn_shells<KM, 1>(P, F, c, u, K, 0, bd, bi, tie, kd, consider, [] {});
+    const bool block = knn_shells<KM, 1>(P, F, c, u, K, 0, bd, bi, tie, kd, consider, [] {});
 #pragma unroll
     for (int j = 0; j < KM; j++)
       if (j < K) P.ind[(long long)j * S + s] = (bd[j] <= 1e32f) ? bi[j] : -1;
+    *knn_left(P, qi) = block && !tie && kd <= 1e32f ? kd : -1.0f;
     if (tie) P.tie_list[atomicAdd(P.knn_ctl, 1)] = (int)s;
   }
 }
@@ -1507,42 +1829,62 @@ __device__ inline void scan_replay(const DevPtrs& P, const KOpts& O, const Frame
   }
 }
 
-// Supervoxels whose K-th distance was tied (listed by the kNN search): their
-// set as the reference's scan keeps it, one wave per listed supervoxel,
+// The set of supervoxel s as the reference's scan keeps it, by one wave,
 // written in the search's (distance, index) order, as every other
 // supervoxel's: the E-step's sums then do not depend on which supervoxels
 // were searched again (the reference's slot layout is formed once, after the
 // last iteration).
 template <int KM>
-__global__ __launch_bounds__(64) void k_knn_exact(DevPtrs P, KOpts O, int words_cap) {
-  extern __shared__ unsigned long long bits[];
-  const int cnt = P.knn_ctl[0];
+__device__ inline void knn_replay(const DevPtrs& P, const KOpts& O, const FrameDev* F,
+                                  long long s, int words_cap, unsigned long long* bits) {
   const long long S = P.Scap;
   const int K = O.K;
+  const float q0 = P.sv_cent[s], q1 = P.sv_cent[S + s], q2 = P.sv_cent[2 * S + s];
+  ScanSlotsOne<KM> sl;
+  scan_replay<KM, true>(P, O, F, true, q0, q1, q2, words_cap, bits, sl);
+  if (threadIdx.x == 0) {
+    float od[KM];
+    int oi[KM];
+#pragma unroll
+    for (int j = 0; j < KM; j++) {
+      od[j] = INFINITY;
+      oi[j] = 0x7fffffff;
+    }
+    bool unused = false;
+    float kd = INFINITY;
+#pragma unroll
+    for (int j = 0; j < KM; j++)
+      if (j < K && sl.mi[j] >= 0) knn_try<KM>(od, oi, sl.dist(j), sl.mi[j], K, unused, kd);
+#pragma unroll
+    for (int j = 0; j < KM; j++)
+      if (j < K) P.ind[(long long)j * S + s] = od[j] <= 1e32f ? (int)(F->g0 + oi[j]) : -1;
+  }
+  __syncthreads();  // the bitmap is free for the next supervoxel
+}
+
+// What the search left, one wave each: the queries that a look found to need
+// a new search (and a replay, if their K-th distance is tied then), and the
+// tied supervoxels of the full search. kFewBlocks blocks where a look can list
+// many.
+constexpr int kFewBlocks = 2048;
+
+template <int KM>
+__global__ __launch_bounds__(64) void k_knn_exact(DevPtrs P, KOpts O, int words_cap) {
+  extern __shared__ unsigned long long bits[];
+  const int cnt = P.knn_ctl[0], few = P.knn_ctl[3];
+  for (int t = blockIdx.x; t < few; t += gridDim.x) {
+    const long long i = P.pairs[t];
+    const FrameDev* F = P.fr + P.sblk_frame[i >> 8];
+    const bool tie = knn_wave<KM>(P, O, F, i, reinterpret_cast<int*>(bits + words_cap));
+    __syncthreads();  // the rows' places are free
+    if (tie) {
+      if (threadIdx.x == 0) atomicAdd(P.knn_ctl + 4, 1);
+      knn_replay<KM>(P, O, F, __float_as_int(P.q4[i].w), words_cap, bits);
+    }
+  }
   for (int t = blockIdx.x; t < cnt; t += gridDim.x) {
     const long long s = P.tie_list[t];
-    const FrameDev* F = P.fr + P.sv_frame[s];
-    const float q0 = P.sv_cent[s], q1 = P.sv_cent[S + s], q2 = P.sv_cent[2 * S + s];
-    ScanSlotsOne<KM> sl;
-    scan_replay<KM, true>(P, O, F, true, q0, q1, q2, words_cap, bits, sl);
-    if (threadIdx.x == 0) {
-      float od[KM];
-      int oi[KM];
-#pragma unroll
-      for (int j = 0; j < KM; j++) {
-        od[j] = INFINITY;
-        oi[j] = 0x7fffffff;
-      }
-      bool unused = false;
-      float kd = INFINITY;
-#pragma unroll
-      for (int j = 0; j < KM; j++)
-        if (j < K && sl.mi[j] >= 0) knn_try<KM>(od, oi, sl.dist(j), sl.mi[j], K, unused, kd);
-#pragma unroll
-      for (int j = 0; j < KM; j++)
-        if (j < K) P.ind[(long long)j * S + s] = od[j] <= 1e32f ? (int)(F->g0 + oi[j]) : -1;
-    }
-    __syncthreads();  // the bitmap is free for the next listed supervoxel
+    knn_replay<KM>(P, O, P.fr + P.sv_frame[s], s, words_cap, bits);
   }
 }
 
@@ -1575,7 +1917,7 @@ __global__ __launch_bounds__(64) void k_knn_layout(DevPtrs P, KOpts O, int only_
   const float4 qq = in ? P.q4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   const long long s = in ? __float_as_int(qq.w) : 0;
   // the row of grid cells of the lane's query
-  const int row = in ? (int)((P.qcell[s] - F->c0) / F->dims[0]) : 0x7fffffff;
+  const int row = in ? (int)((P.qcell[i] - F->c0) / F->dims[0]) : 0x7fffffff;
   ScanSlots<KM> sl;
 #pragma unroll
   for (int j = 0; j < KM; j++) {
@@ -1868,13 +2210,6 @@ __global__ __launch_bounds__(256) void k_pair_scatter(DevPtrs P, KOpts O) {
   }
 }
 
-// Orders of the LDS accesses of one wave's lanes (no block barrier).
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Pair lists written out in order of code (= of supervoxel), so that the FP64
 // accumulation order is fixed. A Gaussian's runs (k_pair_scatter) hold
 // disjoint ranges of supervoxels (a supervoxel lists a Gaussian at most
@@ -2079,7 +2414,7 @@ __device__ inline double alpha_after(const DevPtrs& P, long long k, bool live, d
 }
 
 // Posterior (GMEM.cu:1601-1677) and regularisation (GMEM.cu:1693-1809) of
-// Gaussian k from its M-step sums (mst), if it is alive and not fixed;
+// Gaussian k from its M-step sums (msums), if it is alive and not fixed;
 // commits this iteration's E[ln det] and E[ln pi].
 __device__ inline GaussState posterior_one(const DevPtrs& P, const KOpts& O, long long k,
                                            double psi_sum) {
@@ -2095,7 +2430,14 @@ __device__ inline GaussState posterior_one(const DevPtrs& P, const KOpts& O, lon
   for (int i = 0; i < 3; i++) g.m[i] = gsv(P, GS_M + i, k);
   for (int i = 0; i < 6; i++) g.W[i] = gsv(P, GS_W + i, k);
   const bool live = g.alive && !g.fixed;
-  const double N = P.mst[k];
+  double st[10];
+#pragma unroll
+  for (int i = 0; i < 5; i++) {
+    const double2 v = msums(P, k)[i];
+    st[2 * i] = v.x;
+    st[2 * i + 1] = v.y;
+  }
+  const double N = st[0];
   g.nu = nu_after(P, k, live, N);
   g.alpha = alpha_after(P, k, live, N);
   if (!live) {
@@ -2103,8 +2445,8 @@ __device__ inline GaussState posterior_one(const DevPtrs& P, const KOpts& O, lon
     return g;
   }
   double S1[3], S2[6];
-  for (int i = 0; i < 3; i++) S1[i] = P.mst[(1 + i) * G + k];
-  for (int i = 0; i < 6; i++) S2[i] = P.mst[(4 + i) * G + k];
+  for (int i = 0; i < 3; i++) S1[i] = st[1 + i];
+  for (int i = 0; i < 6; i++) S2[i] = st[4 + i];
   double xk[3] = {0, 0, 0}, Ck[6] = {0, 0, 0, 0, 0, 0};
   if (N > 0.0) {
     const double m0 = S1[0] / N, m1 = S1[1] / N, m2 = S1[2] / N;
@@ -2327,7 +2669,8 @@ __global__ __launch_bounds__(64 * ML) void k_mstep(DevPtrs P, KOpts O) {
   if (threadIdx.x >= 64) return;
   const long long k = (long long)blockIdx.x * 64 + threadIdx.x;
 #pragma unroll
-  for (int i = 0; i < 10; i++) P.mst[i * G + k] = sums[i][threadIdx.x];
+  for (int i = 0; i < 5; i++)
+    msums(P, k)[i] = make_double2(sums[2 * i][threadIdx.x], sums[2 * i + 1][threadIdx.x]);
   double alpha = 0.0;
   if (P.g_frame[k] == f)
     alpha = alpha_after(P, k, gsv(P, GS_M_O, k) > -1e31 && P.fixed[k] == 0,
@@ -2373,7 +2716,7 @@ __global__ __launch_bounds__(256) void k_death(DevPtrs P, KOpts O) {
     if (mine) g = posterior_one(P, O, k, F->psi_sum_alpha);
   } else if (mine) {
     const bool live = gsv(P, GS_M_O, k) > -1e31 && P.fixed[k] == 0;
-    const double N = P.mst[k];
+    const double N = msums(P, k)[0].x;
     const double nu = nu_after(P, k, live, N);
     if (w == 1) {
       psi_s[0][l] = digamma(0.5 * (nu + 1.0 - 0));
@@ -3082,6 +3425,11 @@ static void launch_mstep(const DevPtrs& P, const KOpts& O, hipStream_t st) {
 
 template <int KM>
 static void launch_knn(const DevPtrs& P, const KOpts& O, hipStream_t st) {
+  if (O.tiles.knn_lanes == 64) {
+    k_knn_small<KM><<<nb(P.Sext, 4), 256, 0, st>>>(P, O);
+    return;
+  }
+  k_knn_look<<<nb(P.Sext, 256), 256, 0, st>>>(P, O);
   if (O.tiles.knn_lanes == 0) {  // one block of knn_block/64 waves per grid cell
     const unsigned g = (unsigned)P.Cext;
     if (O.tiles.knn_block == 64)
@@ -3141,13 +3489,14 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
   const unsigned gb = nb(P.Gext, kGB);
   const int bs = O.tiles.sv_block;
   k_scan_frames<<<P.nframes, 1024, 0, st>>>(P, 0, 1, O.K);
-  k_grid_scatter<<<gb, kGB, 0, st>>>(P);
+  k_grid_scatter<<<gb, kGB, 0, st>>>(P, O);
   if (tk == TK_KNN && e0) (void)hipEventRecord(e0, st);
   launch_knn<KM>(P, O, st);
   if (tk == TK_KNN && e1) (void)hipEventRecord(e1, st);
   {
     const int words = (int)std::min<long long>(kLayoutWords, (P.Gext + 63) / 64);
-    k_knn_exact<KM><<<128, 64, scan_lds_bytes(words), st>>>(P, O, words);
+    k_knn_exact<KM><<<O.tiles.knn_lanes == 64 ? 128 : kFewBlocks, 64, scan_lds_bytes(words), st>>>(
+        P, O, words);
   }
   if (tk == TK_ESTEP && e0) (void)hipEventRecord(e0, st);
   k_estep<KM><<<nb(P.Sext, bs), bs, 0, st>>>(P, O);

@@ -119,6 +119,8 @@ int ws_alloc(Workspace* w, const WsShape& sh, int K) {
   AL(P.qcell_start, C + 1);
   AL(P.cblk_frame, C / kCB + 1);
   AL(P.cg4, G);
+  AL(P.cell_mv, C + 1);
+  AL(P.mv_pos, (long long)kMovedCap * C);
   AL(P.mknn, G);
   AL(P.tie_list, S);
   AL(P.knn_ctl, 64);
@@ -128,7 +130,6 @@ int ws_alloc(Workspace* w, const WsShape& sh, int K) {
   AL(P.svkeep, 17 * G);
   AL(P.part_g, G / kGB);
   AL(P.part_g2, G / kGB);
-  AL(P.mst, 10 * G);
   AL(P.part_s, S / kLLminB);
   AL(P.part_sg, S / 256);
   AL(P.fr, F);
@@ -145,9 +146,9 @@ void ws_free(Workspace* w) {
 
 long long ws_bytes_estimate(const WsShape& sh, int K) {
   const long long S = sh.Scap, G = sh.Gcap, C = sh.Ccap, V = sh.Vcap;
-  return 24 * V + S * (16 + 8 + 4 + 12 + 80 + 80 + 12 + 16 + 17LL * K + 1 + 4 + 8) +
+  return 24 * V + S * (16 + 8 + 4 + 12 + 80 + 80 + 12 + 16 + 16LL * K + 1 + 4 + 8) +
          G * (4 + 8 * GS_NFIELDS * 2 + 1 + 96 + 8 + 64 + 12 + 4 + 8 + 12 + 4 + 1 + 16 + 288 +
-              68 + 4 + 4 + 80) +
+              68 + 4) +
          8 * C + 64 * sh.Fcap;
 }
 
@@ -197,13 +198,46 @@ KOpts make_kopts(const tgmm_em_opts& o, const float* scale_reg) {
   k.lmin = o.lambda_min;
   k.lmax = o.lambda_max;
   k.emax = o.max_excentricity;
-  k.tiles = kDefaultTiles;
   k.voxel = o.voxel_mode ? 1 : 0;
-  if (k.voxel) {  // the log-likelihood's lane-per-voxel form
-    k.tiles.ll_gw = 1;
-    k.tiles.ll_u = 1;
-  }
+  k.tiles = tiles_for(0, 1, o.K, k.voxel != 0);
   return k;
+}
+
+// Each line lies where the measured times of the two sides cross (us):
+//   M-step lanes 4 / 8 / 16 by the mean pair list S / G: 1.7 pairs 20 / 34 /
+//     46 (153,000 Gaussians), 4.2 pairs 8.4 / 9.6 / 10.7 (200), 10.6 pairs 15.4
+//     / 11.0 / 12.5 (10,000), 11.1 pairs 34 / 26.5 / 28.8 (60,000), 485 pairs
+//     (per-voxel, 10,000) 98 / 65 / 49;
+//   log-likelihood in blocks of 16 supervoxels, two voxels a thread, against
+//     32 and four, where there are blocks to fill the chip: 128 / 140 (668,000
+//     supervoxels), 52 / 55 (270,000), 27.0 / 26.7 (109,000), 10.2 / 9.5 (900);
+//   kNN lanes per query 1 / 2 / 4: 145 / 170 / 240 (668,000 supervoxels, K = 8),
+//     385 / 570 / 965 (4.9M one-voxel queries), 68 / 65 / 70 (200,000), 71 / 57 /
+//     52 (60,000, K = 8), 33 / 25.5 / 23 (25,000); a wave per query on the
+//     smallest batches: 6.2 against 16.5 with 2 lanes (900).
+Tiles tgmm::tiles_for(long long S, long long G, int K, bool voxel) {
+  Tiles t = kDefaultTiles;
+  if (S >= 6 * G)
+    t.ms_lanes = S >= 32 * G ? 16 : 8;
+  else
+    t.ms_lanes = 4;
+  if (voxel) {  // the log-likelihood's lane-per-voxel form
+    t.ll_gw = 1;
+    t.ll_u = 1;
+  } else if (S >= 131072 && K <= 8) {
+    t.ll_gw = 64;
+    t.ll_u = 2;
+  }
+  if (S <= 16384) {
+    t.knn_lanes = 64;
+  } else if (S <= 65536) {
+    t.knn_lanes = 4;
+    t.knn_block = 64;
+  } else if (S >= 300000) {
+    t.knn_lanes = 1;
+    t.knn_block = 64;
+  }
+  return t;
 }
 
 bool tgmm::tiles_valid(const Tiles& t) {
@@ -213,7 +247,7 @@ bool tgmm::tiles_valid(const Tiles& t) {
          in(t.ms_lanes, 4, 8, 16) &&
          in(t.sv_block, 64, 128, 256) && in(t.knn_block, 64, 128, 256) &&
          (t.knn_chunk == 4 || t.knn_chunk == 8) && in(t.knn_cell, 2, 4, 6) &&
-         (t.knn_lanes == 0 || in(t.knn_lanes, 1, 2, 4));
+         (t.knn_lanes == 0 || t.knn_lanes == 64 || in(t.knn_lanes, 1, 2, 4));
 }
 
 // records (AoS, host) -> 27 x G SoA columns at [g0, g0+G) of a Gcap table,
@@ -369,6 +403,7 @@ int batch_build(int device, const std::vector<FrameSrc>& fs_in, const tgmm_em_op
   P.Sext = need.Scap;
   P.Gext = need.Gcap;
   P.Cext = need.Ccap;
+  b->ko.tiles = tiles_for(s, g, o.K, o.voxel_mode != 0);
   int rc = batch_upload(b, fs);
   if (rc) {
     tgmm_batch_destroy(b);
@@ -654,10 +689,10 @@ extern "C" int tgmm_batch_fetch(tgmm_batch* b, tgmm_frame_desc* frames, int nfra
 extern "C" int tgmm_batch_stats(tgmm_batch* b, tgmm_batch_stats_t* st) {
   if (!b || !st) return TGMM_ERR_ARG;
   HIPCHK(hipSetDevice(b->device));
-  int ctl[2] = {0, 0};
+  int ctl[5] = {0, 0, 0, 0, 0};
   HIPCHK(hipMemcpyAsync(ctl, b->ws.P.knn_ctl, sizeof(ctl), hipMemcpyDeviceToHost, b->st));
   HIPCHK(hipStreamSynchronize(b->st));
-  st->knn_ties_last_iteration = ctl[0];
+  st->knn_ties_last_iteration = ctl[0] + ctl[4];
   st->layout_mismatches = ctl[1];
   st->workspace_bytes = b->ws.bytes;
   return TGMM_OK;
@@ -833,6 +868,7 @@ extern "C" int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, 
     int n;
     int v[15][3];
   };
+  const bool small = b->ws.P.Sext <= 65536;  // a wave per query is tried too
   const Knob knobs[5] = {
       {"loglik", TK_LOGLIK, 10, {{16, 1}, {16, 2}, {16, 4}, {16, 8}, {32, 1}, {32, 2}, {32, 4},
                                  {64, 1}, {64, 2}, {64, 4}}},
@@ -841,7 +877,8 @@ extern "C" int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, 
       {"knn_cell", TK_KNN, 3, {{2, 0}, {4, 0}, {6, 0}}},
       {"knn", TK_KNN, 15, {{64, 8, 0},  {128, 8, 0}, {256, 8, 0}, {64, 4, 1},  {256, 4, 1},
                            {64, 8, 1},  {256, 8, 1}, {64, 4, 2},  {256, 4, 2}, {64, 8, 2},
-                           {256, 8, 2}, {64, 4, 4},  {256, 4, 4}, {64, 8, 4},  {256, 8, 4}}},
+                           {256, 8, 2}, {64, 4, 4},  {256, small ? 8 : 4, small ? 64 : 4}, {64, 8, 4},
+                           {256, 8, 4}}},
   };
   int rc = TGMM_OK;
   for (int q = 0; q < 5 && rc == TGMM_OK; q++) {

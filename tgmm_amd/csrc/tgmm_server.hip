@@ -202,6 +202,7 @@ struct tgmm_server {
   std::vector<long long> to_download;   // retired this step, copies not yet queued
   tgmm_server_opts o;
   KOpts ko;
+  bool user_tiles = false;  // launch shapes set by the caller
   Workspace ws;
   RangeAlloc av, as, ag, ac;
   std::vector<int> slot_ticket;
@@ -440,6 +441,8 @@ static int update_extents(tgmm_server* s) {
   P.Sext = std::min(se, P.Scap);
   P.Gext = std::min(ge, P.Gcap);
   P.Cext = std::min(ce, P.Ccap);
+  if (!s->user_tiles)  // (knn_cell stays: the grids in flight were built with it)
+    s->ko.tiles = tiles_for(P.Sext, P.Gext, s->o.em.K, false);
   if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
   if (s->graph) (void)hipGraphDestroy(s->graph);
   s->gexec = nullptr;
@@ -1024,6 +1027,7 @@ extern "C" int tgmm_server_set_tiles(tgmm_server* s, const tgmm_tiles* t) {
   if (int rc = drain(s)) return rc;
   HIPCHK(hipStreamSynchronize(s->st));
   s->ko.tiles = x;
+  s->user_tiles = true;
   if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
   if (s->graph) (void)hipGraphDestroy(s->graph);
   s->gexec = nullptr;
