@@ -1608,53 +1608,98 @@ __device__ inline void scan_box(ScanBox& b, const SlotsOf<KM, ONE>& sl, bool liv
 }
 
 // Up to 64 Gaussians, one a lane (index k relative to the frame, -1 past the
-// end, in increasing order over the lanes), through the scan.
-template <int KM, bool ONE>
-__device__ inline void scan_take64(SlotsOf<KM, ONE>& sl, const ScanBox& box, float q0, float q1,
-                                   float q2, float4 r, int k, float s0, float s1, float s2,
-                                   int K) {
+// end, in increasing order over the lanes), through the scan of the wave's
+// one query: the lanes that pass the current threshold, lowest index first,
+// the test repeated after every insertion.
+template <int KM>
+__device__ inline void scan_take64(ScanSlotsOne<KM>& sl, float q0, float q1, float q2, float4 r,
+                                   int k, float s0, float s1, float s2, int K) {
   const int lane = threadIdx.x & 63;
   const bool ok = k >= 0 && !(r.x != r.x);  // in range and alive
-  if constexpr (ONE) {
+  float p1, p2, d;
+  ScanSlots<KM>::terms(q0, q1, q2, r, s0, s1, s2, p1, p2, d);
+  unsigned long long mask = __ballot(ok && sl.passes(p1, p2, d));
+  while (mask) {
+    const int u = __builtin_ctzll(mask);
+    sl.insert(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), u)),
+              __builtin_amdgcn_readlane(k, u), K);
+    mask = __ballot(ok && lane > u && sl.passes(p1, p2, d));
+  }
+}
+
+// n <= 64 collected Gaussians (in LDS, in index order) through the scan of
+// each lane's query: a lane marks, branch-free, those not above its threshold
+// at the start (a superset of the ones its scan takes, since the threshold
+// only falls; a NaN distance is marked) and walks its marks in order with the
+// exact test. The wave then pays for its busiest lane's marks, not for every
+// Gaussian that any lane takes.
+template <int KM>
+__device__ inline void scan_marked(ScanSlots<KM>& sl, const float4* got, int n, float q0,
+                                   float q1, float q2, float s0, float s1, float s2, int K) {
+  unsigned long long cand = 0ull;
+  const float t0 = sl.thr;
+  for (int b = 0; b < n; b += 8) {
+    unsigned m = 0u;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      float p1, p2, d;
+      ScanSlots<KM>::terms(q0, q1, q2, got[b + u], s0, s1, s2, p1, p2, d);
+      m |= d > t0 ? 0u : 1u << u;
+    }
+    cand |= (unsigned long long)m << b;
+  }
+  const unsigned long long all = n < 64 ? (1ull << n) - 1ull : ~0ull;
+  cand &= all;
+  while (cand) {
+    const int u = __builtin_ctzll(cand);
+    cand &= cand - 1ull;
+    const float4 r = got[u];
     float p1, p2, d;
     ScanSlots<KM>::terms(q0, q1, q2, r, s0, s1, s2, p1, p2, d);
-    unsigned long long mask = __ballot(ok && sl.passes(p1, p2, d));
-    while (mask) {
-      const int u = __builtin_ctzll(mask);
-      sl.insert(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), u)),
-                __builtin_amdgcn_readlane(k, u), K);
-      mask = __ballot(ok && lane > u && sl.passes(p1, p2, d));
-    }
-  } else {
-    bool in = ok;
-    if (!box.wide) {  // comparisons with NaN keep the Gaussian
-      const double u0 = (double)r.x * s0, u1 = (double)r.y * s1, u2 = (double)r.z * s2;
-      in = in && !(u0 < box.lo[0] || u0 > box.hi[0] || u1 < box.lo[1] || u1 > box.hi[1] ||
-                   u2 < box.lo[2] || u2 > box.hi[2]);
-    }
-    unsigned long long mask = __ballot(in);
-    while (mask) {
-      const int u = __builtin_ctzll(mask);
-      mask &= mask - 1ull;
-      float4 ru;
-      ru.x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.x), u));
-      ru.y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.y), u));
-      ru.z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.z), u));
-      ru.w = 0.0f;
-      sl.take(q0, q1, q2, ru, __builtin_amdgcn_readlane(k, u), s0, s1, s2, K);
-    }
+    if (!sl.passes(p1, p2, d)) continue;
+    sl.insert(d, __float_as_int(r.w), K);
+    // a NaN threshold takes the next Gaussian, whatever its distance
+    if (sl.thr != sl.thr && u + 1 < 64) cand |= (~0ull << (u + 1)) & all;
+  }
+}
+
+// The 64 Gaussians r (index k, in: inside the box) broadcast to the lanes'
+// queries one after another.
+template <int KM>
+__device__ inline void scan_each(ScanSlots<KM>& sl, bool in, float4 r, int k, float q0, float q1,
+                                 float q2, float s0, float s1, float s2, int K) {
+  unsigned long long mask = __ballot(in);
+  while (mask) {
+    const int u = __builtin_ctzll(mask);
+    mask &= mask - 1ull;
+    float4 ru;
+    ru.x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.x), u));
+    ru.y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.y), u));
+    ru.z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.z), u));
+    ru.w = 0.0f;
+    sl.take(q0, q1, q2, ru, __builtin_amdgcn_readlane(k, u), s0, s1, s2, K);
   }
 }
 
 // n Gaussians through the scan, 64 * U per round (U loads a lane issued
 // together), the box refreshed every round. idx(i) is the i-th Gaussian's
-// frame-relative index (increasing in i).
+// frame-relative index (increasing in i). ONE = false: of those inside the box
+// of the wave's balls, with up to 5 slots, 64 are collected in LDS (got, 64 *
+// (U + 1) entries) and marked at a time; with more slots a walk over marks
+// costs as much as the insertions it saves, and its LDS takes places on the CU
+// (60,000 Gaussians, K = 8: 655 us each in turn, 780 marked; K = 5: 10,000
+// Gaussians 168 and 137, 32 frames 870 and 680, 4.9M one-voxel queries 1790
+// and 1520).
+constexpr int kScanU = 4;
+constexpr bool scan_marks(int km) { return km <= 5; }
+
 template <int KM, bool ONE, class Idx>
 __device__ inline void scan_list(const float4* mk, int n, Idx idx, SlotsOf<KM, ONE>& sl, ScanBox& box,
                                  bool live, float q0, float q1, float q2, float s0, float s1,
-                                 float s2, int K) {
-  constexpr int U = ONE ? 8 : 4;  // loads a lane in flight
+                                 float s2, int K, float4* got) {
+  constexpr int U = ONE ? 8 : kScanU;  // loads a lane in flight
   const int lane = threadIdx.x & 63;
+  int held = 0;
   for (int b = 0; b < n; b += 64 * U) {
     float4 r[U];
     int kk[U];
@@ -1664,16 +1709,57 @@ __device__ inline void scan_list(const float4* mk, int n, Idx idx, SlotsOf<KM, O
       kk[c] = i < n ? idx(i) : -1;
       r[c] = kk[c] >= 0 ? mk[kk[c]] : make_float4(NAN, 0.f, 0.f, 0.f);
     }
+    if constexpr (ONE) {
 #pragma unroll
-    for (int c = 0; c < U; c++)
-      if (b + 64 * c < n) scan_take64<KM, ONE>(sl, box, q0, q1, q2, r[c], kk[c], s0, s1, s2, K);
+      for (int c = 0; c < U; c++)
+        if (b + 64 * c < n) scan_take64<KM>(sl, q0, q1, q2, r[c], kk[c], s0, s1, s2, K);
+    } else {
+#pragma unroll
+      for (int c = 0; c < U; c++) {
+        if (b + 64 * c >= n) continue;
+        bool in = kk[c] >= 0 && !(r[c].x != r[c].x);  // in range and alive
+        if (!box.wide) {  // comparisons with NaN keep the Gaussian
+          const double u0 = (double)r[c].x * s0, u1 = (double)r[c].y * s1,
+                       u2 = (double)r[c].z * s2;
+          in = in && !(u0 < box.lo[0] || u0 > box.hi[0] || u1 < box.lo[1] || u1 > box.hi[1] ||
+                       u2 < box.lo[2] || u2 > box.hi[2]);
+        }
+        if constexpr (scan_marks(KM)) {
+          const unsigned long long m = __ballot(in);
+          if (in)
+            got[held + (int)__builtin_amdgcn_mbcnt_hi(
+                           (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
+                make_float4(r[c].x, r[c].y, r[c].z, __int_as_float(kk[c]));
+          held += __popcll(m);
+        } else {
+          scan_each<KM>(sl, in, r[c], kk[c], q0, q1, q2, s0, s1, s2, K);
+        }
+      }
+      if constexpr (scan_marks(KM)) {
+        wave_lds_sync();
+        int at = 0;
+        // the last round takes what is left; before it, whole 64s
+        const bool last = b + 64 * U >= n;
+        for (; at + 64 <= held || (last && at < held); at += 64)
+          scan_marked<KM>(sl, got + at, min(64, held - at), q0, q1, q2, s0, s1, s2, K);
+        held = max(held - at, 0);
+        if (at > 0 && held > 0) {  // the Gaussians left move to the front
+          const float4 rest = got[at + (lane < held ? lane : 0)];
+          wave_lds_sync();
+          if (lane < held) got[lane] = rest;
+        }
+      }
+    }
     scan_box<KM, ONE>(box, sl, live);
   }
 }
 
 // dynamic LDS of a kernel calling scan_replay with words_cap = words
-inline size_t scan_lds_bytes(int words) {
-  return (size_t)std::max(words, 1) * 8 + (size_t)kListCap * sizeof(int);
+// (rounded so that the collected Gaussians after it are 16-byte aligned)
+inline int scan_words(int words) { return (std::max(words, 1) + 1) & ~1; }
+inline size_t scan_lds_bytes(int words, bool marks) {
+  return (size_t)words * 8 + (size_t)kListCap * sizeof(int) +
+         (marks ? (size_t)64 * (kScanU + 1) * sizeof(float4) : 0);
 }
 
 template <int KM, bool ONE>
@@ -1687,6 +1773,7 @@ __device__ inline void scan_replay(const DevPtrs& P, const KOpts& O, const Frame
   const float s0 = O.scale[0], s1 = O.scale[1], s2 = O.scale[2];
   const float4* mk = P.mknn + g0;
   int* list = reinterpret_cast<int*>(bits + words_cap);
+  float4* got = reinterpret_cast<float4*>(list + kListCap);
   sl.init(live);
   ScanBox box;
   for (int a = 0; a < 3; a++) {
@@ -1718,7 +1805,7 @@ __device__ inline void scan_replay(const DevPtrs& P, const KOpts& O, const Frame
     const int m2 = min(ng, m + (ONE ? 512 : 256));
     const int mb = m;
     scan_list<KM, ONE>(mk, m2 - mb, [mb](int i) { return mb + i; }, sl, box, live, q0, q1, q2,
-                       s0, s1, s2, K);
+                       s0, s1, s2, K, got);
     m = m2;
     if (m >= ng) break;
     if (!box.wide) {
@@ -1738,7 +1825,7 @@ __device__ inline void scan_replay(const DevPtrs& P, const KOpts& O, const Frame
   if (box.wide || words > words_cap || ncell > kLayoutCells) {
     const int mb = m;
     scan_list<KM, ONE>(mk, ng - mb, [mb](int i) { return mb + i; }, sl, box, live, q0, q1, q2,
-                       s0, s1, s2, K);
+                       s0, s1, s2, K, got);
     return;
   }
   for (int w = lane; w < words; w += 64) bits[w] = 0ull;
@@ -1824,7 +1911,7 @@ __device__ inline void scan_replay(const DevPtrs& P, const KOpts& O, const Frame
     }
     __syncthreads();
     scan_list<KM, ONE>(mk, min(kListCap, tot - base), [list](int i) { return list[i]; }, sl, box,
-                       live, q0, q1, q2, s0, s1, s2, K);
+                       live, q0, q1, q2, s0, s1, s2, K, got);
     __syncthreads();  // the list is rewritten next
   }
 }
@@ -1888,6 +1975,53 @@ __global__ __launch_bounds__(64) void k_knn_exact(DevPtrs P, KOpts O, int words_
   }
 }
 
+// The search's candidates of supervoxel s into the reference's slots mi
+// (frame-relative Gaussians), and its candidate with r > 0.5.
+template <int KM>
+__device__ inline void layout_write(const DevPtrs& P, long long g0, int K, long long s,
+                                    const int (&mi)[KM]) {
+  const long long S = P.Scap;
+  int oi[KM];
+  float orr[KM];
+  // one round of loads (a slot past K reads row 0, not used): no load
+  // waits for the previous slot's
+#pragma unroll
+  for (int j = 0; j < KM; j++) {
+    const long long row = j < K ? j : 0;
+    const int ij = P.ind[row * S + s];
+    const float rj = P.rnk[row * S + s];
+    oi[j] = j < K ? ij : -1;
+    orr[j] = j < K ? rj : 0.0f;
+  }
+  int n_old = 0, n_new = 0;
+#pragma unroll
+  for (int j = 0; j < KM; j++) {
+    n_old += (j < K && oi[j] >= 0) ? 1 : 0;
+    n_new += (j < K && mi[j] >= 0) ? 1 : 0;
+  }
+  bool same = n_old == n_new;
+  int2 w = make_int2(-1, -1);
+#pragma unroll
+  for (int j = 0; j < KM; j++) {
+    if (j >= K) continue;
+    const int k = mi[j] >= 0 ? (int)(g0 + mi[j]) : -1;
+    float r = 0.0f;
+    bool found = k < 0;
+#pragma unroll
+    for (int t = 0; t < KM; t++)
+      if (t < K && k >= 0 && oi[t] == k) {
+        r = orr[t];
+        found = true;
+      }
+    same &= found;
+    P.ind[(long long)j * S + s] = k;
+    P.rnk[(long long)j * S + s] = r;
+    if (k >= 0 && r > 0.5f) w = make_int2(k, j);
+  }
+  P.win[s] = w;
+  if (!same) atomicAdd(P.knn_ctl + 1, 1);
+}
+
 // The slot layout of every supervoxel after a solve: the reference's scan of
 // its last kNN search replayed exactly (scan_replay), 64 supervoxels of
 // one frame in grid-cell order per wave. The wave's supervoxels are replayed
@@ -1924,58 +2058,39 @@ __global__ __launch_bounds__(64) void k_knn_layout(DevPtrs P, KOpts O, int only_
     sl.md[j] = 1e32f;
     sl.mi[j] = -1;
   }
+  // (with no more Gaussians than the first phase scans anyway, all at once)
   bool todo = in;
+  const bool once = F->ng <= 1024;
   while (__any(todo)) {
-    int r0 = todo ? row : 0x7fffffff;  // the lowest row left
+    int r0 = todo ? (once ? 0 : row) : 0x7fffffff;  // the lowest row left
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) r0 = min(r0, __shfl_xor(r0, o, 64));
-    const bool live = todo && row == r0;
+    const bool live = todo && (once || row == r0);
     scan_replay<KM, false>(P, O, F, live, qq.x, qq.y, qq.z, words_cap, bits, sl);
     __syncthreads();  // the bitmap and list are free for the next row
     todo = todo && !live;
   }
-  if (in) {
-    // the search's candidates into the reference's slots
-    int oi[KM];
-    float orr[KM];
-    // one round of loads (a slot past K reads row 0, not used): no load
-    // waits for the previous slot's
-#pragma unroll
-    for (int j = 0; j < KM; j++) {
-      const long long row = j < K ? j : 0;
-      const int ij = P.ind[row * S + s];
-      const float rj = P.rnk[row * S + s];
-      oi[j] = j < K ? ij : -1;
-      orr[j] = j < K ? rj : 0.0f;
-    }
-    int n_old = 0, n_new = 0;
-#pragma unroll
-    for (int j = 0; j < KM; j++) {
-      n_old += (j < K && oi[j] >= 0) ? 1 : 0;
-      n_new += (j < K && sl.mi[j] >= 0) ? 1 : 0;
-    }
-    bool same = n_old == n_new;
-    int2 w = make_int2(-1, -1);
-#pragma unroll
-    for (int j = 0; j < KM; j++) {
-      if (j >= K) continue;
-      const int k = sl.mi[j] >= 0 ? (int)(g0 + sl.mi[j]) : -1;
-      float r = 0.0f;
-      bool found = k < 0;
-#pragma unroll
-      for (int t = 0; t < KM; t++)
-        if (t < K && k >= 0 && oi[t] == k) {
-          r = orr[t];
-          found = true;
-        }
-      same &= found;
-      P.ind[(long long)j * S + s] = k;
-      P.rnk[(long long)j * S + s] = r;
-      if (k >= 0 && r > 0.5f) w = make_int2(k, j);
-    }
-    P.win[s] = w;
-    if (!same) atomicAdd(P.knn_ctl + 1, 1);
-  }
+  if (in) layout_write<KM>(P, g0, K, s, sl.mi);
+}
+
+// The same with a wave per supervoxel, for up to kLayoutOne of them: 64
+// Gaussians at a time against one query, every query at once (a lane per query
+// leaves most of the chip idle then). 900 supervoxels 148 -> 12.4 us, 16,500
+// 111 -> 74; 24,500 126 against 117 here.
+constexpr long long kLayoutOne = 24576;
+template <int KM>
+__global__ __launch_bounds__(64) void k_knn_layout_one(DevPtrs P, KOpts O, int only_frame,
+                                                       int words_cap) {
+  extern __shared__ unsigned long long bits[];
+  const long long i = P.s_lo + blockIdx.x;
+  const int f = P.sblk_frame[i >> 8];
+  if (f < 0 || (only_frame >= 0 && f != only_frame)) return;
+  const FrameDev* F = P.fr + f;
+  if (F->iter <= 1 || F->ng <= 0 || i >= F->s0 + F->ns) return;  // no kNN ran
+  const float4 q = P.q4[i];
+  ScanSlotsOne<KM> sl;
+  scan_replay<KM, true>(P, O, F, true, q.x, q.y, q.z, words_cap, bits, sl);
+  if (threadIdx.x == 0) layout_write<KM>(P, F->g0, O.K, __float_as_int(q.w), sl.mi);
 }
 
 // The returned records (GaussianMixtureModelCUDA, 288 bytes), one lane per
@@ -3457,9 +3572,14 @@ static void launch_knn(const DevPtrs& P, const KOpts& O, hipStream_t st) {
 template <int KM>
 static void launch_knn_layout_t(const DevPtrs& P, const KOpts& O, int only_frame, int max_ng,
                                 hipStream_t st) {
-  const int words = (int)std::min<long long>(kLayoutWords, ((long long)max_ng + 63) / 64);
-  k_knn_layout<KM><<<nb(P.Sext, 64), 64, scan_lds_bytes(words), st>>>(P, O, only_frame,
-                                                                               words);
+  const int words =
+      scan_words((int)std::min<long long>(kLayoutWords, ((long long)max_ng + 63) / 64));
+  if (P.Sext <= kLayoutOne)
+    k_knn_layout_one<KM><<<(unsigned)P.Sext, 64, scan_lds_bytes(words, false), st>>>(
+        P, O, only_frame, words);
+  else
+    k_knn_layout<KM><<<nb(P.Sext, 64), 64, scan_lds_bytes(words, scan_marks(KM)), st>>>(
+        P, O, only_frame, words);
 }
 
 hipError_t launch_knn_layout(const DevPtrs& P, const KOpts& O, int only_frame, int max_ng,
@@ -3494,9 +3614,9 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
   launch_knn<KM>(P, O, st);
   if (tk == TK_KNN && e1) (void)hipEventRecord(e1, st);
   {
-    const int words = (int)std::min<long long>(kLayoutWords, (P.Gext + 63) / 64);
-    k_knn_exact<KM><<<O.tiles.knn_lanes == 64 ? 128 : kFewBlocks, 64, scan_lds_bytes(words), st>>>(
-        P, O, words);
+    const int words = scan_words((int)std::min<long long>(kLayoutWords, (P.Gext + 63) / 64));
+    k_knn_exact<KM><<<O.tiles.knn_lanes == 64 ? 128 : kFewBlocks, 64, scan_lds_bytes(words, false),
+                      st>>>(P, O, words);
   }
   if (tk == TK_ESTEP && e0) (void)hipEventRecord(e0, st);
   k_estep<KM><<<nb(P.Sext, bs), bs, 0, st>>>(P, O);
