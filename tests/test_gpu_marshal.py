@@ -145,3 +145,24 @@ def test_batch_from_raw_frames_equals_batch_from_host_arrays():
         assert records_equal(g["gm"], w["gm"])
         assert np.array_equal(g["rnk"], w["rnk"]) and np.array_equal(g["ind"], w["ind"])
         assert g["ll"] == w["ll"] and g["iterations"] == w["iterations"]
+
+
+@pytest.mark.parametrize("dims", [(65535, 65537, 1), (65536, 65536, 1), (4294967295, 1, 1),
+                                  (1, 1, 4294967296), (3, 2147483659, 7), (1, 4000000007, 1)])
+def test_coordinates_around_32_bits(dims):
+    """Indices at the ends and at row boundaries, on both sides of the volume
+    size where the division changes its width; lists of 0 to 49 voxels, around
+    one and several rows of 16."""
+    rng = np.random.default_rng(dims[0] % 1000)
+    vol = dims[0] * dims[1] * dims[2]
+    lens = np.array([0, 1, 15, 16, 17, 31, 32, 33, 48, 49, 0])
+    n = int(lens.sum())
+    edge = [0, vol - 1] + [v for m in (1, 2, vol // dims[0]) for v in
+                           (m * dims[0] - 1, m * dims[0] % vol, (m * dims[0] + 1) % vol)]
+    idx = np.concatenate([np.array(edge, np.uint64) % np.uint64(vol),
+                          rng.integers(0, vol, n - len(edge), dtype=np.uint64)])
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    args = (idx, rng.integers(0, 65536, n).astype(np.uint16), ptr,
+            rng.integers(0, 3000, len(lens)).astype(np.uint16), np.array(dims, np.int64))
+    print("marshal dims %s" % (dims,), flush=True)
+    _same(_gpu(*args), O.marshal_frame(*args))

@@ -13,7 +13,7 @@
 //                (uint16 arithmetic, as the reference's unsigned short), the
 //                centroid of the raw intensities accumulated in float in list
 //                order (each lane forms its voxel's products; the group adds
-//                them in order through shuffles, with no contraction), and
+//                them in order from its lanes, with no contraction), and
 //                per block the range of the subtracted image;
 //   k_mar_range  one block: the image range from the block partials;
 //   k_mar_scale  lane per voxel: Scale_Array_To_Range(img, 0, 1) over the
@@ -55,6 +55,22 @@ __device__ inline unsigned long long div_exact(unsigned long long n, unsigned lo
   return q;
 }
 
+// The same in 32 bits, for n < 2^32 and d < 2^32: the double product is exact
+// The same for n and d below 2^32.
+__device__ inline unsigned div_exact32(unsigned n, unsigned d, double inv, unsigned& r) {
+  unsigned q = (unsigned)((double)n * inv);
+  long long rem = (long long)n - (long long)((unsigned long long)q * d);
+  if (rem < 0) {
+    q -= 1;
+    rem += d;
+  } else if (rem >= (long long)d) {
+    q += 1;
+    rem -= d;
+  }
+  r = (unsigned)rem;
+  return q;
+}
+
 __global__ void k_mar_init(unsigned* range) {
   if (threadIdx.x == 0) range[2] = 0u;  // set when an index lies outside the volume
 }
@@ -90,6 +106,34 @@ __global__ __launch_bounds__(1024) void k_mar_range(const unsigned* __restrict__
   }
 }
 
+// v of lane j of the 16-lane row, in every lane of it (one DPP operand of the
+// instruction that uses it)
+template <int J>
+__device__ inline float row_lane(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + J, 0xf, 0xf, true));
+}
+
+// The row's 16 voxels added in list order; lanes past the end add +0.0, which
+// leaves the (non-negative) sums unchanged.
+template <int J = 0>
+__device__ inline void add_row(float w, float px, float py, float pz, float& nk, float& cx,
+                               float& cy, float& cz) {
+#pragma clang fp contract(off)
+  nk += row_lane<J>(w);
+  cx += row_lane<J>(px);
+  cy += row_lane<J>(py);
+  cz += row_lane<J>(pz);
+  if constexpr (J + 1 < kMG) add_row<J + 1>(w, px, py, pz, nk, cx, cy, cz);
+}
+
+// The list's four sums, in its order, are 4 dependent additions a voxel: they
+// are 64 instructions per 16 voxels, each reading its addend from another
+// lane of the row (through shuffles they were 64 LDS permutes more, and the
+// kernel 73 us for 4.9M voxels in 110,000 supervoxels; now 41, 127 MB). The
+// next 16 voxels are loaded before the current ones are added. SMALL: the
+// volume has fewer than 2^32 voxels, and the coordinates are split in 32 bits.
+template <bool SMALL>
 __global__ __launch_bounds__(kMB) void k_mar_sv(
     const unsigned long long* __restrict__ idx, const unsigned short* __restrict__ raw,
     const unsigned short* __restrict__ volume, const long long* __restrict__ ptr,
@@ -106,42 +150,55 @@ __global__ __launch_bounds__(kMB) void k_mar_sv(
     const long long beg = ptr[s], end = ptr[s + 1];
     const unsigned short th = thr[s];
     float nk = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
+    unsigned long long id = 0;
+    unsigned short r = 0;
+    auto load = [&](long long v) {  // voxel v's index and intensity
+      id = 0;
+      r = 0;
+      if (v < end) {
+        id = idx[v];
+        if (raw) r = raw[v];
+        else if (id < vol) r = volume[id];
+      }
+    };
+    load(beg + lane);
     for (long long base = beg; base < end; base += kMG) {  // the same trips in a group
       const long long v = base + lane;
       float w = 0.0f, px = 0.0f, py = 0.0f, pz = 0.0f;
+      const unsigned long long id_v = id;
+      unsigned short r_v = r;
+      load(v + kMG);
       if (v < end) {
-        const unsigned long long id = idx[v];
-        unsigned long long x = 0, y = 0, z = 0;
-        unsigned short r = 0;
-        if (id >= vol) {
+        float x = 0.0f, y = 0.0f, z = 0.0f;
+        if (id_v >= vol) {
           bad = 1u;
+          r_v = 0;
+        } else if constexpr (SMALL) {
+          unsigned xi, yi;
+          const unsigned q = div_exact32((unsigned)id_v, (unsigned)d0, inv0, xi);
+          z = (float)div_exact32(q, (unsigned)d1, inv1, yi);
+          x = (float)xi;
+          y = (float)yi;
         } else {
-          const unsigned long long q = div_exact(id, d0, inv0, x);
-          z = div_exact(q, d1, inv1, y);
-          r = raw ? raw[v] : volume[id];
+          unsigned long long xi, yi;
+          const unsigned long long q = div_exact(id_v, d0, inv0, xi);
+          z = (float)div_exact(q, d1, inv1, yi);
+          x = (float)xi;
+          y = (float)yi;
         }
-        query[v] = (float)x;
-        query[v + N] = (float)y;
-        query[v + 2 * N] = (float)z;
-        const unsigned short sub = (unsigned short)(r - th);
+        query[v] = x;
+        query[v + N] = y;
+        query[v + 2 * N] = z;
+        const unsigned short sub = (unsigned short)(r_v - th);
         img[v] = (float)sub;
         hi = sub > hi ? sub : hi;
         lo = sub < lo ? sub : lo;
-        w = (float)r;
-        px = w * (float)x;
-        py = w * (float)y;
-        pz = w * (float)z;
+        w = (float)r_v;
+        px = w * x;
+        py = w * y;
+        pz = w * z;
       }
-      // the chunk's voxels in list order; lanes past the end add +0.0,
-      // which leaves the (non-negative) sums unchanged
-#pragma unroll
-      for (int j = 0; j < kMG; j++) {
-#pragma clang fp contract(off)
-        nk += __shfl(w, j, kMG);
-        cx += __shfl(px, j, kMG);
-        cy += __shfl(py, j, kMG);
-        cz += __shfl(pz, j, kMG);
-      }
+      add_row(w, px, py, pz, nk, cx, cy, cz);
     }
     if (lane == 0) {
       const bool zero = (double)nk < 1e-5;
@@ -270,14 +327,15 @@ int marshal_run(const tgmm_raw_frame* f, const unsigned long long* idx, const un
                           0)) != hipSuccess)
     return hip_fail(e, "copy of the supervoxel pointer");
   k_mar_init<<<1, 64, 0, 0>>>(range);
+  const unsigned long long voxels = (unsigned long long)f->dims[0] *
+                                    (unsigned long long)f->dims[1] *
+                                    (unsigned long long)f->dims[2];
   if (S > 0)
-    k_mar_sv<<<nsb, kMB, 0, 0>>>(
+    (voxels <= 0xffffffffull ? k_mar_sv<true> : k_mar_sv<false>)<<<nsb, kMB, 0, 0>>>(
         idx, raw, f->volume, ptr, thr, S, N, (unsigned long long)f->dims[0],
-        (unsigned long long)f->dims[1],
-        (unsigned long long)f->dims[0] * (unsigned long long)f->dims[1] *
-            (unsigned long long)f->dims[2],
-        1.0 / (double)f->dims[0], 1.0 / (double)f->dims[1], queryCUDA, imgDataCUDA,
-        centroidLabelPositionCUDA, part_hi, part_lo, range);
+        (unsigned long long)f->dims[1], voxels, 1.0 / (double)f->dims[0],
+        1.0 / (double)f->dims[1], queryCUDA, imgDataCUDA, centroidLabelPositionCUDA, part_hi,
+        part_lo, range);
   if (N > 0) k_mar_range<<<1, 1024, 0, 0>>>(part_hi, part_lo, nsb, range);
   const double vol = (double)f->dims[0] * (double)f->dims[1] * (double)f->dims[2];
   if (N > 0)
