@@ -204,6 +204,12 @@ struct DevPtrs {
 // kernel launchers (tgmm_kernels.hip); all enqueue on `st`
 // once per frame: supervoxel moments, kNN grid shape, queries sorted by cell
 hipError_t launch_prep(const DevPtrs& P, const KOpts& O, hipStream_t st);
+// The workspace's range tables from the frame table, every supervoxel's voxel
+// range from its first and past-the-last voxel in the frame (P.sv_beg and
+// P.win as 8-byte integers; voxel: one voxel each), and the state columns
+// (P.gs and gs_init), fixed flags and supervoxel lists from the records given
+// in P.rec.
+hipError_t launch_load(const DevPtrs& P, double* gs_init, int voxel, hipStream_t st);
 // iteration state, initial sum of alpha and first E-step constants per frame;
 // the frames' kNN grid counts must be zero
 hipError_t launch_reset(const DevPtrs& P, const KOpts& O, hipStream_t st);

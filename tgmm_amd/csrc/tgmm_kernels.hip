@@ -2167,6 +2167,83 @@ __global__ __launch_bounds__(256) void k_finalize(DevPtrs P, KOpts O, int cap, i
   }
 }
 
+// The range tables of a workspace whose frames tile it in order (a lane per
+// entry of the longest): which frame a supervoxel, a Gaussian and each of
+// their blocks belongs to (-1: padding), and a supervoxel's voxels. Formed
+// here instead of on the host, where 24,000 supervoxels and 5,500 records
+// took 0.7 ms of filling fresh vectors before the first kernel.
+__global__ __launch_bounds__(256) void k_frame_tables(DevPtrs P, int voxel) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  // the last frame whose range starts at or before i (the first starts at 0,
+  // and no range is empty)
+  auto frame_of = [&](long long FrameDev::*start) {
+    int lo = 0, hi = P.nframes;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (P.fr[mid].*start <= i) lo = mid;
+      else hi = mid;
+    }
+    return lo;
+  };
+  if (i < P.Scap) {
+    const int f = frame_of(&FrameDev::s0);
+    const FrameDev* F = P.fr + f;
+    const long long j = i - F->s0, ns = F->ns;
+    long long beg = 0;
+    int len = 0;
+    if (j < ns && voxel) {
+      beg = F->v0 + j;
+      len = 1;
+    } else if (j < ns) {
+      const long long a = P.sv_beg[i], e = reinterpret_cast<const long long*>(P.win)[i];
+      beg = F->v0 + a;
+      len = (int)(e - a);
+    }
+    P.sv_frame[i] = j < ns ? f : -1;
+    P.sv_beg[i] = beg;
+    P.sv_len[i] = len;
+    if (i % kAlign == 0)
+      P.sblk_frame[i / kAlign] = j < kAlign * (long long)F->nbl ? f : -1;
+  }
+  if (i < P.Gcap) {
+    const int f = frame_of(&FrameDev::g0);
+    const FrameDev* F = P.fr + f;
+    const long long j = i - F->g0;
+    P.g_frame[i] = j < F->ng ? f : -1;
+    if (i % kGB == 0) P.gblk_frame[i / kGB] = j < kGB * (long long)F->nbg ? f : -1;
+  }
+  if (i <= P.Ccap && i % kCB == 0) {
+    const int f = frame_of(&FrameDev::c0);
+    P.cblk_frame[i / kCB] = i - P.fr[f].c0 < P.fr[f].ncap ? f : -1;
+  }
+}
+
+// k_finalize's reverse: the given records into the state columns, the fixed
+// flags and the supervoxel lists (zeros where no Gaussian is), 16 records a
+// block, read in one contiguous piece.
+__global__ __launch_bounds__(256) void k_load_records(DevPtrs P, double* __restrict__ gs_init) {
+  constexpr int kRec = sizeof(GaussianMixtureModelCUDA) / 4;  // 72 words
+  constexpr int kIdx = 55;                                    // supervoxelIdx's first word
+  __shared__ __align__(16) int rec[16 * kRec];
+  const long long k0 = (long long)blockIdx.x * 16, G = P.Gcap;
+  for (int i = threadIdx.x; i < 16 * 18; i += 256) {
+    int4 v = make_int4(0, 0, 0, 0);
+    if (P.g_frame[k0 + i / 18] >= 0) v = reinterpret_cast<const int4*>(P.rec + k0)[i];
+    reinterpret_cast<int4*>(rec)[i] = v;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 16 * GS_NFIELDS; i += 256) {
+    const int field = i >> 4, g = i & 15;
+    const double v = reinterpret_cast<const double*>(rec + g * kRec)[field];
+    P.gs[(long long)field * G + k0 + g] = v;
+    gs_init[(long long)field * G + k0 + g] = v;
+  }
+  for (int i = threadIdx.x; i < 16 * 17; i += 256)
+    P.svkeep[17 * k0 + i] = rec[(i / 17) * kRec + kIdx + i % 17];
+  if (threadIdx.x < 16)  // the flag's byte; the three after it are padding
+    P.fixed[k0 + threadIdx.x] = (rec[threadIdx.x * kRec + 54] & 0xff) != 0;
+}
+
 // Responsibilities of the K candidates of each supervoxel. The reference's
 // per-voxel sum of -0.5(3/beta + nu d^T W d) + E[ln pi] + 0.5 E[ln det]
 // (GMEM.cu:2281-2298) equals, exactly,
@@ -3614,6 +3691,12 @@ hipError_t launch_knn_layout(const DevPtrs& P, const KOpts& O, int only_frame, i
     default:
       launch_knn_layout_t<16>(P, O, only_frame, max_ng, st);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_load(const DevPtrs& P, double* gs_init, int voxel, hipStream_t st) {
+  k_frame_tables<<<nb(std::max(std::max(P.Scap, P.Gcap), P.Ccap + 1), 256), 256, 0, st>>>(P, voxel);
+  k_load_records<<<nb(P.Gcap, 16), 256, 0, st>>>(P, gs_init);
   return hipGetLastError();
 }
 

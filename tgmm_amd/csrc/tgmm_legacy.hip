@@ -352,6 +352,7 @@ extern "C" int tgmm_GMEMvariationalInferenceCUDAWithSupervoxels(
   f.img = imgDataCUDA;
   f.cent = centroidLabelPositionCUDA;
   f.ptr = ptr.data();
+  f.ptr_dev = labelListPtrCUDA;
   f.gm = vecGMtemp;
   return run_frame(devCUDA, f, o, sreg, vecGMtemp, rnkCUDA, indCUDA, indCUDAtr, S, debugPath,
                    frame);

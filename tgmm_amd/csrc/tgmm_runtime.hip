@@ -283,20 +283,14 @@ int batch_build(int device, const std::vector<FrameSrc>& fs_in, const tgmm_em_op
   // voxel mode (GMEMupdateCUDA.cu:3420-3973): every voxel is its own kNN
   // query and a one-voxel supervoxel whose centroid is the voxel itself
   std::vector<FrameSrc> vfs;
-  std::vector<std::vector<long long>> vptr;
   if (o.voxel_mode) {
     vfs = fs_in;
-    vptr.resize(fs_in.size());
     for (size_t i = 0; i < fs_in.size(); i++) {
       if (fs_in[i].N < 0) {
         tgmm_set_error("frame %zu: negative size", i);
         return TGMM_ERR_ARG;
       }
-      vptr[i].resize(fs_in[i].N + 1);
-      for (long long v = 0; v <= fs_in[i].N; v++) vptr[i][v] = v;
       vfs[i].S = fs_in[i].N;
-      vfs[i].cent = fs_in[i].query;
-      vfs[i].ptr = vptr[i].data();
     }
   }
   const std::vector<FrameSrc>& fs = o.voxel_mode ? vfs : fs_in;
@@ -418,15 +412,9 @@ int batch_upload(tgmm_batch* b, const std::vector<FrameSrc>& fs) {
   const WsShape& sh = b->ws.sh;
   hipStream_t st = b->st;
   const long long S = sh.Scap, G = sh.Gcap;
-  std::vector<int> sv_frame(S, -1), sv_len(S, 0), g_frame(G, -1);
-  std::vector<long long> sv_beg(S, 0);
-  std::vector<int> sblk(S / kAlign, -1), gblk(G / kGB, -1), cblk(b->ws.sh.Ccap / kCB + 1, -1);
-  std::vector<double> gs((size_t)GS_NFIELDS * G, 0.0);
-  std::vector<unsigned char> fixed(G, 0);
-  std::vector<int> svkeep((size_t)17 * G, 0);
-  for (size_t i = 0; i < fs.size(); i++) {
+  const bool voxel = b->opts.voxel_mode != 0;
+  for (size_t i = 0; i < fs.size() && !voxel; i++) {
     const FrameSrc& f = fs[i];
-    const FrameDev& F = b->fh[i];
     for (long long j = 0; j < f.S; j++) {
       const long long a = f.ptr[j], e = f.ptr[j + 1];
       if (a < 0 || e < a || e > f.N) {
@@ -437,17 +425,10 @@ int batch_upload(tgmm_batch* b, const std::vector<FrameSrc>& fs) {
         tgmm_set_error("frame %zu: supervoxel with more than 2^31 voxels", i);
         return TGMM_ERR_LIMIT;
       }
-      sv_frame[F.s0 + j] = (int)i;
-      sv_beg[F.s0 + j] = F.v0 + a;
-      sv_len[F.s0 + j] = (int)(e - a);
     }
-    for (long long j = 0; j < round_up(std::max<long long>(f.S, 1), kAlign) / kAlign; j++)
-      sblk[F.s0 / kAlign + j] = (int)i;
-    for (long long j = 0; j < F.nbg; j++) gblk[F.g0 / kGB + j] = (int)i;
-    for (long long j = 0; j < F.ncap / kCB; j++) cblk[F.c0 / kCB + j] = (int)i;
-    for (long long k = 0; k < f.G; k++) g_frame[F.g0 + k] = (int)i;
-    if (f.G > 0) records_to_soa(f.gm, f.G, F.g0, G, gs.data(), fixed.data(), svkeep.data());
   }
+  // The caller's arrays go up as they are; the range tables and the state
+  // columns are formed from them on the device (launch_load).
   const hipMemcpyKind kv = hipMemcpyDefault;
   for (size_t i = 0; i < fs.size(); i++) {
     const FrameSrc& f = fs[i];
@@ -458,24 +439,26 @@ int batch_upload(tgmm_batch* b, const std::vector<FrameSrc>& fs) {
       HIPCHK(hipMemcpyAsync(P.vz + F.v0, f.query + 2 * f.N, f.N * 4, kv, st));
       HIPCHK(hipMemcpyAsync(P.vimg + F.v0, f.img, f.N * 4, kv, st));
     }
-    if (f.S > 0)
+    if (f.S > 0 && voxel) {  // the centroids are the voxels
+      const float* v[3] = {P.vx, P.vy, P.vz};
+      for (int a = 0; a < 3; a++)
+        HIPCHK(hipMemcpyAsync(P.sv_cent + a * S + F.s0, v[a] + F.v0, f.S * 4,
+                              hipMemcpyDeviceToDevice, st));
+    } else if (f.S > 0) {
       for (int a = 0; a < 3; a++)
         HIPCHK(hipMemcpyAsync(P.sv_cent + a * S + F.s0, f.cent + a * f.S, f.S * 4, kv, st));
+      // where each supervoxel begins and ends
+      const long long* ptr = f.ptr_dev ? f.ptr_dev : f.ptr;
+      HIPCHK(hipMemcpyAsync(P.sv_beg + F.s0, ptr, f.S * 8, kv, st));
+      HIPCHK(hipMemcpyAsync(P.win + F.s0, ptr + 1, f.S * 8, kv, st));
+    }
+    if (f.G > 0)
+      HIPCHK(hipMemcpyAsync(P.rec + F.g0, f.gm, f.G * sizeof(GaussianMixtureModelCUDA), kv, st));
   }
-  HIPCHK(hipMemcpyAsync(P.sv_frame, sv_frame.data(), S * 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.sv_beg, sv_beg.data(), S * 8, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.sv_len, sv_len.data(), S * 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.sblk_frame, sblk.data(), sblk.size() * 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.cblk_frame, cblk.data(), cblk.size() * 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.g_frame, g_frame.data(), G * 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.gblk_frame, gblk.data(), gblk.size() * 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.gs, gs.data(), gs.size() * 8, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(b->ws.gs_init, gs.data(), gs.size() * 8, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.fixed, fixed.data(), G, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(P.svkeep, svkeep.data(), svkeep.size() * 4, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemsetAsync(P.knn_ctl, 0, 64 * 4, st));
   HIPCHK(hipMemcpyAsync(P.fr, b->fh.data(), b->fh.size() * sizeof(FrameDev), hipMemcpyHostToDevice,
                         st));
+  HIPCHK(launch_load(P, b->ws.gs_init, voxel ? 1 : 0, st));
   HIPCHK(hipMemsetAsync(P.ind, 0xFF, (size_t)b->ws.K * S * 4, st));
   HIPCHK(hipMemsetAsync(P.rnk, 0, (size_t)b->ws.K * S * 4, st));
   HIPCHK(hipMemsetAsync(P.seg_cnt, 0, (G + 1) * 4, st));

@@ -23,7 +23,8 @@ struct Workspace {
 };
 
 // One frame's inputs: pointers may be host or device memory (copied with
-// hipMemcpyDefault); ptr and gm are host memory.
+// hipMemcpyDefault); ptr and gm are host memory. ptr and cent are not read in
+// voxel mode; ptr_dev, if given, is a device copy of ptr.
 struct FrameSrc {
   long long N = 0, S = 0;
   int G = 0;
@@ -31,6 +32,7 @@ struct FrameSrc {
   const float* img = nullptr;
   const float* cent = nullptr;
   const long long* ptr = nullptr;
+  const long long* ptr_dev = nullptr;
   const GaussianMixtureModelCUDA* gm = nullptr;
 };
 
