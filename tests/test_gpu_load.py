@@ -53,3 +53,18 @@ def test_frames_around_range_ends(shift, voxel):
         if f.N > 0:
             e = record_errors(got["gm"], gm_o)
             assert max(e.values()) < 1e-5, e
+
+
+@pytest.mark.parametrize("G", [4095, 4096, 8193, 33000])
+def test_scans_around_a_segment(G):
+    """The scans of cells and pair lists at one segment of 4,096 entries, one
+    entry more, several, and a second pass of eight, beside a small frame."""
+    small, f = _frame(3, 64, seed=1), _frame(G, 1500, seed=G)
+    print("scan G=%d" % G, flush=True)
+    with em.Batch([small, f], em.make_opts(max_iter=3)) as b:
+        b.solve(em.SOLVE_GRAPH)
+        got = b.fetch()[1]
+    gm_o, rnk_o, ind_o, hist, it, ll = O.em_run(f, O.make_opts(max_iter=3))
+    assert np.array_equal(got["ind"], ind_o)
+    e = record_errors(got["gm"], gm_o)
+    assert max(e.values()) < 1e-5, e

@@ -161,6 +161,7 @@ struct DevPtrs {
   // grid
   int* cell_cnt;    // Ccap+1
   int* cell_start;  // Ccap+1
+  int* cell_next;   // Ccap+1: the next search's cell_start, until its scatter
   int* qcell_start; // Ccap+1: first kNN query of each cell (positions in q4)
   int* cblk_frame;  // Ccap/kCB: frame of each 64-cell block, -1 if none
   float4* cg4;      // Gcap: cell-sorted references (x, y, z, index bits)

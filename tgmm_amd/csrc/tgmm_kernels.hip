@@ -434,6 +434,27 @@ __global__ __launch_bounds__(kGB) void k_alpha_init(DevPtrs P) {
   if (threadIdx.x == 0) P.part_g[gb] = t;
 }
 
+// A frame's sum of alpha from the Gaussian-block partials of the kernel
+// before, by one wave, partials in index order (lane l takes l, l+64,
+// ... into four interleaved sums, then a fixed butterfly): the sum used by
+// E[ln pi] and the log-likelihood, with its digamma and log.
+__device__ inline void alpha_sum_frame(const DevPtrs& P, int block, int need_active) {
+  const int f = (P.only_frame >= 0) ? P.only_frame : block;
+  if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
+  FrameDev* F = P.fr + f;
+  if (F->ncap == 0 || (need_active && !F->active)) return;
+  const double tot = frame_sum_w64(P.part_g + F->g0 / kGB, F->nbg);
+  if (threadIdx.x == 0) {
+    F->sum_alpha = tot;
+    F->psi_sum_alpha = digamma(tot);
+    F->log_sum_alpha = log(tot);
+  }
+}
+
+__global__ __launch_bounds__(64) void k_alpha_sum(DevPtrs P, int need_active) {
+  alpha_sum_frame(P, (int)blockIdx.x, need_active);
+}
+
 // ---------------------------------------------------------------- scans --
 constexpr int kSortShort = 128;  // longer pair lists are listed for the block-wide sort
 constexpr int kScanQ = 8;        // int4 loads per thread and pass, k_scan_frames (4 | kScanQ)
@@ -449,57 +470,44 @@ constexpr int kSortLds = 4096;   // longest list sorted in LDS
 //            positions of the frame's queries in cell order).
 // Both ranges hold n+1 entries (the grid has fewer cells than its range, the
 // Gaussian range at least one padding entry), so frames never share an entry.
-// A pass covers kScanQ segments of 4096 entries; in segment q thread t loads
+// A pass covers Q segments of 4096 entries; in segment q thread t loads
 // and stores entries 4t .. 4t+3 as one int4 (consecutive threads, consecutive
 // 16 bytes: a wave's load touches 8 cache lines, where a contiguous run per
 // thread touched 64), and the ranges start on multiples of 4. The prefix of
 // an int4 is the carry, the sums of the pass's earlier segments, and the sums
-// of the segment's earlier threads: one wave scan per segment, the
-// (segment, wave) totals scanned by wave 0.
-__global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int need_active,
-                                                      int K) {
-  constexpr int NW = 16;  // waves per block
-  static_assert(kScanQ % 4 == 0, "whole values per lane in the totals scan");
-  __shared__ int wsum[kScanQ * NW];
-  __shared__ int total;
-  // the grid scan opens an iteration: the kNN's tie list starts empty
-  if (which == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
-    P.knn_ctl[0] = 0;
-    P.knn_ctl[2] = 0;  // and the list of long pair lists
-    P.knn_ctl[3] = 0;  // and the queries to search for again
-    P.knn_ctl[4] = 0;
-  }
-  const int f = (P.only_frame >= 0) ? P.only_frame : (int)blockIdx.x;
-  if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
-  const FrameDev* F = P.fr + f;
-  if (F->ncap == 0 || (need_active && !F->active)) return;  // empty slot / finished
-  if (which == 0 && threadIdx.x == 0) P.fr[f].moved = 0;
-  const int* in;
-  int* out;
-  long long n;
-  int base;
-  if (which == 0 || which == 2) {
-    in = P.cell_cnt + F->c0;
-    out = (which == 0 ? P.cell_start : P.qcell_start) + F->c0;
-    n = (long long)F->dims[0] * F->dims[1] * F->dims[2];
-    base = (int)(which == 0 ? F->g0 : F->s0);
-  } else {
-    in = P.seg_cnt + F->g0;
-    out = P.seg_start + F->g0;
-    n = F->ng;
-    base = (int)(K * F->s0);
-  }
+// of the segment's earlier threads: one wave scan per segment (additions
+// whose operand is another lane's, no LDS), the (segment, wave) totals
+// scanned by wave 0. A frame of one segment takes it alone: eight side by
+// side, most of them empty, cost it 7.4 us instead of 3.3 (200
+// Gaussians), a latency chain of two loads, the scans and a store.
+__device__ inline int wave_scan_incl(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast 15, 31
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+
+// which: the kind of scan, F its frame, k_scan_frames' arguments.
+template <int Q>
+__device__ inline void scan_frame(const DevPtrs& P, const FrameDev* F, int which, const int* in,
+                                  int* out, long long n, int base, int* wsum, int& total) {
+  constexpr int NW = 16;                                    // waves per block
+  constexpr int PL = Q * NW / 64 > 0 ? Q * NW / 64 : 1;     // totals per lane of wave 0
+  static_assert(PL * 64 == Q * NW || Q == 1, "whole values per lane in the totals scan");
   const long long n1 = n + 1;  // entry n carries the total
   // the pair scan lists the Gaussians whose pair list is long, for the
   // block-wide sort (k_seg_sort)
   const bool list_long = which == 1;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int carry = base;
-  for (long long c0 = 0; c0 < n1; c0 += 4096LL * kScanQ) {
-    int4 v[kScanQ];
-    int x[kScanQ], sq[kScanQ];
+  for (long long c0 = 0; c0 < n1; c0 += 4096LL * Q) {
+    int4 v[Q];
+    int x[Q], sq[Q];
 #pragma unroll
-    for (int q = 0; q < kScanQ; q++) {
+    for (int q = 0; q < Q; q++) {
       const long long e = c0 + 4096LL * q + 4LL * threadIdx.x;
       // the grid scan also clears the moved-mean counts of the frame's cells
       // (a range has a multiple of 64 entries, more than n)
@@ -515,9 +523,8 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
       }
     }
 #pragma unroll
-    for (int q = 0; q < kScanQ; q++) {
+    for (int q = 0; q < Q; q++) {
       sq[q] = v[q].x + v[q].y + v[q].z + v[q].w;
-      x[q] = sq[q];
       if (list_long && (v[q].x > kSortShort || v[q].y > kSortShort || v[q].z > kSortShort ||
                         v[q].w > kSortShort)) {
         const long long e = c0 + 4096LL * q + 4LL * threadIdx.x;
@@ -527,45 +534,33 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
           if (c[i] > kSortShort) P.long_list[atomicAdd(P.knn_ctl + 2, 1)] = (int)(F->g0 + e + i);
       }
     }
-    // inclusive wave scans, the segments side by side
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-#pragma unroll
-      for (int q = 0; q < kScanQ; q++) {
-        const int y = __shfl_up(x[q], o, 64);
-        if (lane >= o) x[q] += y;
-      }
-    }
+    for (int q = 0; q < Q; q++) x[q] = wave_scan_incl(sq[q]);
     if (lane == 63)
 #pragma unroll
-      for (int q = 0; q < kScanQ; q++) wsum[q * NW + w] = x[q];
+      for (int q = 0; q < Q; q++) wsum[q * NW + w] = x[q];
     __syncthreads();
     if (w == 0) {
-      // the kScanQ * NW totals in (segment, wave) order, PL per lane
-      constexpr int PL = kScanQ * NW / 64;
+      // the Q * NW totals in (segment, wave) order, PL per lane
       int a[PL], y = 0;
 #pragma unroll
       for (int i = 0; i < PL; i++) {
-        a[i] = wsum[PL * lane + i];
+        a[i] = PL * lane + i < Q * NW ? wsum[PL * lane + i] : 0;
         y += a[i];
       }
       const int own = y;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(y, o, 64);
-        if (lane >= o) y += t;
-      }
+      y = wave_scan_incl(y);
       int ex = y - own;
 #pragma unroll
       for (int i = 0; i < PL; i++) {
-        wsum[PL * lane + i] = ex;
+        if (PL * lane + i < Q * NW) wsum[PL * lane + i] = ex;
         ex += a[i];
       }
       if (lane == 63) total = y;
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < kScanQ; q++) {
+    for (int q = 0; q < Q; q++) {
       const long long e = c0 + 4096LL * q + 4LL * threadIdx.x;
       int4 r;
       r.x = carry + wsum[q * NW + w] + x[q] - sq[q];
@@ -583,6 +578,47 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
     carry += total;
     __syncthreads();  // wsum and total are rewritten by the next pass
   }
+}
+
+// Scan 0 follows the binning of the means for the next iteration (k_death,
+// k_gauss_prep). Blocks past the frames' (an iteration has them) form the
+// frames' sums of alpha, which wait for the same kernel and nothing else: one
+// launch instead of two. The search's grid (cell_start) still belongs to the
+// last search, whose slot layout may yet be replayed, so the scan goes to
+// cell_next and k_grid_scatter takes it over.
+__global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int need_active,
+                                                      int K) {
+  __shared__ int wsum[kScanQ * 16];
+  __shared__ int total;
+  const int nscan = P.only_frame >= 0 ? 1 : P.nframes;
+  if ((int)blockIdx.x >= nscan) {
+    if (threadIdx.x < 64) alpha_sum_frame(P, (int)blockIdx.x - nscan, need_active);
+    return;
+  }
+  const int f = (P.only_frame >= 0) ? P.only_frame : (int)blockIdx.x;
+  if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
+  const FrameDev* F = P.fr + f;
+  if (F->ncap == 0 || (need_active && !F->active)) return;  // empty slot / finished
+  if (which == 0 && threadIdx.x == 0) P.fr[f].moved = 0;
+  const int* in;
+  int* out;
+  long long n;
+  int base;
+  if (which == 0 || which == 2) {
+    in = P.cell_cnt + F->c0;
+    out = (which == 0 ? P.cell_next : P.qcell_start) + F->c0;
+    n = (long long)F->dims[0] * F->dims[1] * F->dims[2];
+    base = (int)(which == 0 ? F->g0 : F->s0);
+  } else {
+    in = P.seg_cnt + F->g0;
+    out = P.seg_start + F->g0;
+    n = F->ng;
+    base = (int)(K * F->s0);
+  }
+  if (n < 4096)
+    scan_frame<1>(P, F, which, in, out, n, base, wsum, total);
+  else
+    scan_frame<kScanQ>(P, F, which, in, out, n, base, wsum, total);
 }
 
 // ------------------------------------------------------- iteration kernels --
@@ -662,16 +698,27 @@ __device__ inline void list_moved(const DevPtrs& P, long long cell, float4 m) {
 // not bitwise where the last search saw it is listed in its old cell and in
 // its new one (after the first iteration, which searches for every query).
 __global__ __launch_bounds__(kGB) void k_grid_scatter(DevPtrs P, KOpts O) {
+  // this kernel opens an iteration: the kNN's tie list starts empty
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    P.knn_ctl[0] = 0;
+    P.knn_ctl[2] = 0;  // and the list of long pair lists
+    P.knn_ctl[3] = 0;  // and the queries to search for again
+    P.knn_ctl[4] = 0;
+  }
   const int f = P.gblk_frame[blockIdx.x];
   if (f < 0 || !P.fr[f].active) return;
   const FrameDev* F = P.fr + f;
   const long long k = (long long)blockIdx.x * kGB + threadIdx.x;
+  // the new cells' starts become the search's
+  const long long n1 = (long long)F->dims[0] * F->dims[1] * F->dims[2] + 1;
+  for (long long i = k - F->g0; i < n1; i += (long long)F->nbg * kGB)
+    P.cell_start[F->c0 + i] = P.cell_next[F->c0 + i];
   if (P.g_frame[k] != f) return;
   const float4 m = P.m4[k], old = P.mknn[k];
   P.mknn[k] = m;
   const int c = P.gcell[k];
   if (c >= 0) {
-    const int pos = P.cell_start[c] + atomicSub(P.cell_cnt + c, 1) - 1;
+    const int pos = P.cell_next[c] + atomicSub(P.cell_cnt + c, 1) - 1;
     P.cg4[pos] = m;
   }
   if (F->iter > 1 && (__float_as_int(m.x) != __float_as_int(old.x) ||
@@ -3009,24 +3056,6 @@ __global__ __launch_bounds__(256) void k_death(DevPtrs P, KOpts O) {
   }
 }
 
-// A frame's sum of alpha from the Gaussian-block partials of the kernel
-// before, one wave per frame, partials in index order (lane l takes l, l+64,
-// ... into four interleaved sums, then a fixed butterfly): the sum used by
-// E[ln pi] and the log-likelihood, with its digamma and log.
-__global__ __launch_bounds__(64) void k_alpha_sum(DevPtrs P, int need_active) {
-  const int f = (P.only_frame >= 0) ? P.only_frame : (int)blockIdx.x;
-  if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
-  FrameDev* F = P.fr + f;
-  if (F->ncap == 0 || (need_active && !F->active)) return;
-  const double tot = frame_sum_w64(P.part_g + F->g0 / kGB, F->nbg);
-  if (threadIdx.x == 0) {
-    F->sum_alpha = tot;
-    F->psi_sum_alpha = digamma(tot);
-    F->log_sum_alpha = log(tot);
-  }
-}
-
-
 // Log-likelihood over the voxel stream (GMEM.cu:1913-1978). A block of 256
 // threads takes B consecutive supervoxels of one frame (B divides 256):
 //  1. Candidate constants, LPS lanes per supervoxel (lane j < K: candidate
@@ -3538,6 +3567,7 @@ hipError_t launch_reset(const DevPtrs& P, const KOpts& O, hipStream_t st) {
   k_alpha_init<<<nb(P.Gext, kGB), kGB, 0, st>>>(P);
   k_alpha_sum<<<P.only_frame >= 0 ? 1 : P.nframes, 64, 0, st>>>(P, 1);
   k_gauss_prep<<<nb(P.Gext, kGB), kGB, 0, st>>>(P, O);
+  k_scan_frames<<<P.only_frame >= 0 ? 1 : P.nframes, 1024, 0, st>>>(P, 0, 1, O.K);
   return hipGetLastError();
 }
 
@@ -3711,7 +3741,6 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
                               hipEvent_t e1, int tk) {
   const unsigned gb = nb(P.Gext, kGB);
   const int bs = O.tiles.sv_block;
-  k_scan_frames<<<P.nframes, 1024, 0, st>>>(P, 0, 1, O.K);
   k_grid_scatter<<<gb, kGB, 0, st>>>(P, O);
   if (tk == TK_KNN && e0) (void)hipEventRecord(e0, st);
   launch_knn<KM>(P, O, st);
@@ -3735,7 +3764,7 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
     launch_mstep<false>(P, O, st);
   if (tk == TK_MSTEP && e1) (void)hipEventRecord(e1, st);
   k_death<<<gb, 256, 0, st>>>(P, O);
-  k_alpha_sum<<<P.nframes, 64, 0, st>>>(P, 1);
+  k_scan_frames<<<2 * P.nframes, 1024, 0, st>>>(P, 0, 1, O.K);  // and the sums of alpha
   if (tk == TK_LOGLIK && e0) (void)hipEventRecord(e0, st);
   launch_loglik<KM>(P, O, st, tk == TK_LOGLIK ? e1 : nullptr);
   return hipGetLastError();

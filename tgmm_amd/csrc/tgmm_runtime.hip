@@ -116,6 +116,7 @@ int ws_alloc(Workspace* w, const WsShape& sh, int K) {
   AL(P.pairs_sorted, (long long)K * S);
   AL(P.cell_cnt, C + 1);
   AL(P.cell_start, C + 1);
+  AL(P.cell_next, C + 1);
   AL(P.qcell_start, C + 1);
   AL(P.cblk_frame, C / kCB + 1);
   AL(P.cg4, G);
