@@ -2352,12 +2352,11 @@ __device__ inline void estep_one(const DevPtrs& P, const KOpts& O, long long s, 
     c2 = P.mom[3 * S + s];
 #pragma unroll
     for (int i = 0; i < 6; i++) Q[i] = P.mom[(4 + i) * S + s];
-  } else if (ok) {  // the voxel itself: count 1, no scatter (the same values as mom)
-    const long long v = P.sv_beg[s];
+  } else {  // the voxel itself: count 1, no scatter (the same values as mom)
     n = 1.0;
-    c0 = (double)P.vx[v];
-    c1 = (double)P.vy[v];
-    c2 = (double)P.vz[v];
+    c0 = (double)P.anchor[s];
+    c1 = (double)P.anchor[S + s];
+    c2 = (double)P.anchor[2 * S + s];
 #pragma unroll
     for (int i = 0; i < 6; i++) Q[i] = 0.0;
   }
@@ -2398,7 +2397,7 @@ __device__ inline void estep_one(const DevPtrs& P, const KOpts& O, long long s, 
     }
   }
   // voxel mode stores r times the voxel's intensity (GMEM.cu:2216-2222)
-  const float wv = (ok && O.voxel) ? P.vimg[P.sv_beg[s]] : 1.0f;
+  const float wv = (ok && O.voxel) ? P.vimg[P.fr[f].v0 + (s - P.fr[f].s0)] : 1.0f;
 #pragma unroll
   for (int j = 0; j < KM; j++) {
     if (j < K) {  // K is uniform: the whole wave runs this
@@ -3408,7 +3407,12 @@ __global__ __launch_bounds__(NT) void k_loglik(DevPtrs P, KOpts O) {
 // y = U (x - a) + e = e) over all K candidates (bounding a one-voxel
 // supervoxel's terms costs as much as evaluating them), its supervoxel sum
 // as k_loglik's class sums leave it (0 + term), and the block the same
-// pairwise tree over its 256 supervoxels, without 15 idle lanes of 16.
+// pairwise tree over its 256 supervoxels, without 15 idle lanes of 16. Bound
+// by its loads: the candidates' indices and packs, and 20 bytes a voxel (the
+// anchor, the intensity, the frame); reading the voxel's coordinates, range
+// and length as well, for the same terms, took 114 us instead of 77 on 4.9M
+// voxels. (With the anchor the voxel, U (x - a) is 0, or not finite where e is
+// not either, and such a term is dropped.)
 template <int KM>
 __global__ __launch_bounds__(256) void k_loglik_voxel(DevPtrs P, KOpts O) {
   __shared__ double tree[256];
@@ -3420,11 +3424,9 @@ __global__ __launch_bounds__(256) void k_loglik_voxel(DevPtrs P, KOpts O) {
   const long long s = (long long)blockIdx.x * 256 + threadIdx.x;
   const int K = O.K;
   const double lsa2 = F->log_sum_alpha * 1.4426950408889634074;
-  const int n = (P.sv_frame[s] == f) ? P.sv_len[s] : 0;
   double t = 0.0;
-  if (n > 0) {
-    const long long g = P.sv_beg[s];
-    const float4 vv = make_float4(P.vx[g], P.vy[g], P.vz[g], P.vimg[g]);
+  if (P.sv_frame[s] == f) {
+    const float img = P.vimg[F->v0 + (s - F->s0)];
     const float ca0 = P.anchor[s], ca1 = P.anchor[S + s], ca2 = P.anchor[2 * S + s];
     float tj[KM];
     int nterm = 0;  // candidates with a density (kept by k_loglik's rule in voxel mode)
@@ -3446,12 +3448,7 @@ __global__ __launch_bounds__(256) void k_loglik_voxel(DevPtrs P, KOpts O) {
       nterm += (kk >= 0 && pg > -INFINITY) ? 1 : 0;
       {
 #pragma clang fp contract(off)
-        const float x0 = vv.x - ca0, x1 = vv.y - ca1, x2 = vv.z - ca2;
-        const float y0 = __builtin_fmaf(pu[0], x0, __builtin_fmaf(pu[1], x1,
-                                                                  __builtin_fmaf(pu[2], x2, pe0)));
-        const float y1 = __builtin_fmaf(pu[3], x1, __builtin_fmaf(pu[4], x2, pe1));
-        const float y2 = __builtin_fmaf(pu[5], x2, pe2);
-        const float q = __builtin_fmaf(y0, y0, __builtin_fmaf(y1, y1, y2 * y2));
+        const float q = __builtin_fmaf(pe0, pe0, __builtin_fmaf(pe1, pe1, pe2 * pe2));
         const float tt = pg - q;
         tj[j] = (q <= 1075.0f && tt >= -1075.0f) ? tt : -INFINITY;
       }
@@ -3462,12 +3459,12 @@ __global__ __launch_bounds__(256) void k_loglik_voxel(DevPtrs P, KOpts O) {
 #pragma unroll
       for (int j = 0; j < KM; j++) mx = fmaxf(mx, tj[j]);
       if (nterm == 1) {
-        if (mx > -INFINITY) t = (double)vv.w * (double)mx;
+        if (mx > -INFINITY) t = (double)img * (double)mx;
       } else if (mx > -INFINITY) {
         float sum = 0.0f;
 #pragma unroll
         for (int j = 0; j < KM; j++) sum += __builtin_amdgcn_exp2f(tj[j] - mx);
-        t = (double)vv.w * (double)(mx + __builtin_amdgcn_logf(sum));
+        t = (double)img * (double)(mx + __builtin_amdgcn_logf(sum));
       }
     }
   }
