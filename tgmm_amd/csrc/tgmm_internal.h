@@ -54,6 +54,7 @@ struct FrameDev {
   int active;         // keeps iterating
   int status;
   int moved;          // means that moved since the last kNN search
+  int again;          // queries the look found to search again
   int packed;         // every voxel's offset from its supervoxel's anchor is a
                       // small integer: the log-likelihood reads vpk (set to 1
                       // on the host, cleared by the moments kernel)
@@ -244,7 +245,8 @@ hipError_t launch_finalize(const DevPtrs& P, const KOpts& O, int cap, int only_f
                            int writeback, hipStream_t st);
 
 // timed_kernel ids for launch_iteration
-enum { TK_KNN = 0, TK_ESTEP = 1, TK_MSTEP = 2, TK_LOGLIK = 3 };
+// (TK_SEARCH: the kNN search with what follows it, looks, searches again, ties)
+enum { TK_KNN = 0, TK_ESTEP = 1, TK_MSTEP = 2, TK_LOGLIK = 3, TK_SEARCH = 4 };
 // launches between the timing events: the log-likelihood, which writes only
 // its block partials, runs kTimedLaunches times back to back, so the event
 // pair's own dispatch gap is spread over them; every other kernel updates

@@ -7,20 +7,21 @@
 // Once per frame (launch_prep): per-supervoxel FP64 moments, the frame's
 // uniform kNN grid, and the supervoxel order sorted by grid cell.
 // Per iteration, over all frames of a workspace:
-//   gauss_prep     E[ln det Lambda], E[ln pi] (GMEM.cu:553-628), E-step
-//                  constant, f32 means, kNN grid binning
-//   scan/scatter   counting sort of the means into per-frame grid cells
+//   grid_scatter   counting sort of the means into per-frame grid cells; the
+//                  means that moved since the last search
 //   knn            exact K nearest means per supervoxel centroid by ring
-//                  search (knnCuda.cu:61-144 distance, (dist, idx) order)
+//                  search (knnCuda.cu:61-144 distance, (dist, idx) order);
+//                  where few means moved, only of the queries they concern
 //   estep          responsibilities from per-supervoxel moments
 //                  (GMEM.cu:2244-2336), significant-pair counts
-//   scan/scatter   pairs (s, j) with r > 1e-3 grouped per Gaussian
+//   scan/scatter   pairs (s, j) with r > 1e-3 grouped per Gaussian, by runs
 //   seg_sort       each Gaussian's pair list ordered by supervoxel
-//   mstep_update   FP64 segmented sufficient statistics (GMEM.cu:1286-1455),
-//                  posterior (1601-1677), regularisation (1693-1809),
-//                  per-frame sum of alpha
-//   death          dead-cell rule (1813-1843), log-likelihood parameters,
-//                  per-frame sum of alpha
+//   mstep          FP64 segmented sufficient statistics (GMEM.cu:1286-1455)
+//   death          posterior (1601-1677), regularisation (1693-1809),
+//                  dead-cell rule (1813-1843), log-likelihood parameters,
+//                  E[ln det Lambda], E[ln pi] (553-628), E-step constant, f32
+//                  means and grid binning of the next iteration
+//   scan           the next search's grid cells; per-frame sum of alpha
 //   loglik         voxel stream: img * log sum_k pi_k N(x; m_k, (nu W)^-1)
 //                  (1913-1978), per-frame total, convergence (4145-4148)
 #include <hip/hip_runtime.h>
@@ -599,7 +600,7 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
   if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
   const FrameDev* F = P.fr + f;
   if (F->ncap == 0 || (need_active && !F->active)) return;  // empty slot / finished
-  if (which == 0 && threadIdx.x == 0) P.fr[f].moved = 0;
+  if (which == 0 && threadIdx.x == 0) P.fr[f].moved = P.fr[f].again = 0;
   const int* in;
   int* out;
   long long n;
@@ -1294,6 +1295,15 @@ __device__ inline bool knn_looks(const FrameDev* F) {
   return F->iter > 1 && 128LL * F->moved <= F->ng;
 }
 
+// After the look: whether the queries it listed are searched for by waves, or
+// the frame whole after all. The look cannot clear a query whose K-th
+// neighbour lies outside its block of cells, and with many slots or few means
+// a cell those are many, however few means moved (60,000 Gaussians, K = 8, 2
+// means a cell: 14.2 ms a solve by waves, 13.3 with this rule; 6 a cell: 10.7).
+__device__ inline bool knn_listed(const FrameDev* F) {
+  return knn_looks(F) && 16LL * F->again <= F->ns;
+}
+
 // The look over every query, a lane each: those that may have other neighbours
 // are listed (k_knn_exact searches for them), the others keep the candidates
 // they have. The list lies in the pair runs, which are written later in the
@@ -1312,7 +1322,10 @@ __global__ __launch_bounds__(256) void k_knn_look(DevPtrs P, KOpts O) {
   if (m == 0ull) return;
   const int lane = threadIdx.x & 63;
   int base = 0;
-  if (lane == 0) base = atomicAdd(P.knn_ctl + 3, __popcll(m));
+  if (lane == 0) {
+    base = atomicAdd(P.knn_ctl + 3, __popcll(m));
+    atomicAdd(&P.fr[f].again, __popcll(m));
+  }
   base = __builtin_amdgcn_readfirstlane(base);
   if (need) P.pairs[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)i;
 }
@@ -1327,7 +1340,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KM <= 8 ? 4
   const int f = P.sblk_frame[((long long)blockIdx.x * qpb) >> 8];
   if (f < 0 || !P.fr[f].active) return;
   const FrameDev* F = P.fr + f;
-  if (knn_looks(F)) return;
+  if (knn_listed(F)) return;
   if (i >= F->s0 + F->ns) return;  // the whole group of the query leaves
   knn_search<KM, KC, QL>(P, O, F, i, threadIdx.x % QL, kq);
 }
@@ -1379,7 +1392,7 @@ __global__ __launch_bounds__(64 * NW) void k_knn_cell(DevPtrs P, KOpts O) {
   if (lc >= (long long)nx * ny * nz) return;
   const int qs = P.qcell_start[cc], qe = P.qcell_start[cc + 1];
   if (qs >= qe) return;
-  if (knn_looks(F)) return;
+  if (knn_listed(F)) return;
   const long long c0 = F->c0;
   const int c[3] = {(int)(lc % nx), (int)((lc / nx) % ny), (int)(lc / ((long long)nx * ny))};
   // the 9 rows of the block: lanes 0..8 read the row starts, 9..17 the ends
@@ -2009,6 +2022,7 @@ __global__ __launch_bounds__(64) void k_knn_exact(DevPtrs P, KOpts O, int words_
   for (int t = blockIdx.x; t < few; t += gridDim.x) {
     const long long i = P.pairs[t];
     const FrameDev* F = P.fr + P.sblk_frame[i >> 8];
+    if (!knn_listed(F)) continue;  // searched whole
     const bool tie = knn_wave<KM>(P, O, F, i, reinterpret_cast<int*>(bits + words_cap));
     __syncthreads();  // the rows' places are free
     if (tie) {
@@ -3739,7 +3753,7 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
   const unsigned gb = nb(P.Gext, kGB);
   const int bs = O.tiles.sv_block;
   k_grid_scatter<<<gb, kGB, 0, st>>>(P, O);
-  if (tk == TK_KNN && e0) (void)hipEventRecord(e0, st);
+  if ((tk == TK_KNN || tk == TK_SEARCH) && e0) (void)hipEventRecord(e0, st);
   launch_knn<KM>(P, O, st);
   if (tk == TK_KNN && e1) (void)hipEventRecord(e1, st);
   {
@@ -3747,6 +3761,7 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
     k_knn_exact<KM><<<O.tiles.knn_lanes == 64 ? 128 : kFewBlocks, 64, scan_lds_bytes(words, false),
                       st>>>(P, O, words);
   }
+  if (tk == TK_SEARCH && e1) (void)hipEventRecord(e1, st);
   if (tk == TK_ESTEP && e0) (void)hipEventRecord(e0, st);
   k_estep<KM><<<nb(P.Sext, bs), bs, 0, st>>>(P, O);
   if (tk == TK_ESTEP && e1) (void)hipEventRecord(e1, st);

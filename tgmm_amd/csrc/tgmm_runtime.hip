@@ -858,12 +858,17 @@ extern "C" int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, 
                                  {64, 1}, {64, 2}, {64, 4}}},
       {"mstep", TK_MSTEP, 3, {{4, 0}, {8, 0}, {16, 0}}},
       {"estep", TK_ESTEP, 3, {{64, 0}, {128, 0}, {256, 0}}},
-      {"knn_cell", TK_KNN, 3, {{2, 0}, {4, 0}, {6, 0}}},
-      {"knn", TK_KNN, 15, {{64, 8, 0},  {128, 8, 0}, {256, 8, 0}, {64, 4, 1},  {256, 4, 1},
+      {"knn_cell", TK_SEARCH, 3, {{2, 0}, {4, 0}, {6, 0}}},
+      {"knn", TK_SEARCH, 15, {{64, 8, 0},  {128, 8, 0}, {256, 8, 0}, {64, 4, 1},  {256, 4, 1},
                            {64, 8, 1},  {256, 8, 1}, {64, 4, 2},  {256, 4, 2}, {64, 8, 2},
                            {256, 8, 2}, {64, 4, 4},  {256, small ? 8 : 4, small ? 64 : 4}, {64, 8, 4},
                            {256, 8, 4}}},
   };
+  // The search changes over a solve: whole at first, then only where means
+  // moved, and a grid of small cells suits the first and not the second (60,000
+  // Gaussians, K = 8: 2 means a cell the fastest over 3 iterations, and 14.0 ms
+  // a solve against 10.7 with 6). Its shapes are timed over a whole solve.
+  const int search_iters = std::min(b->opts.max_iter, 32);
   int rc = TGMM_OK;
   for (int q = 0; q < 5 && rc == TGMM_OK; q++) {
     const Knob& kb = knobs[q];
@@ -897,7 +902,8 @@ extern "C" int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, 
           break;
       }
       double ms = 0.0;
-      if ((rc = time_shape(b, t, kb.tk, iters, e0, e1, &ms)) != TGMM_OK) break;
+      if ((rc = time_shape(b, t, kb.tk, q >= 3 ? search_iters : iters, e0, e1, &ms)) != TGMM_OK)
+        break;
       if (q == 4 && kb.v[c][2] == 0)
         snprintf(line, sizeof(line), "%s cell%d %.2f\n", kb.name, kb.v[c][0] / 64, 1000.0 * ms);
       else if (kb.v[c][2])
