@@ -11,5 +11,10 @@ void dm_regularize(double* W, double nu, int w4dof, const float* scale, double l
   tgmm::regularize_W(W, nu, w4dof, scale, lmin, lmax, emax);
 }
 void dm_inv3(const double* w, double* o) { tgmm::inv3(w, o); }
+int dm_look_due(int iter, int blind, long long moved, long long ng) {
+  return tgmm::look_due(iter, blind, moved, ng) ? 1 : 0;
+}
+int dm_look_few(long long listed, long long ns) { return tgmm::look_few(listed, ns) ? 1 : 0; }
+int dm_look_futile(long long stuck, long long ns) { return tgmm::look_futile(stuck, ns) ? 1 : 0; }
 int dm_pair_significant(float r) { return tgmm::pair_significant(r) ? 1 : 0; }
 }

@@ -40,6 +40,23 @@ __host__ __device__ inline double digamma(double x) {
 // is kept.
 __host__ __device__ inline bool pair_significant(float r) { return (double)r > 1e-3; }
 
+// Rules of the kNN search's looks (k_knn_look). A look is due from the second
+// iteration on when at most 1/128 of the frame's ng means moved, unless an
+// earlier one was futile; its list is searched by waves when it holds at most
+// 1/16 of the frame's ns queries (few), else the frame is searched whole; and
+// it was futile when the queries that it has to list whatever moved are past
+// that line by themselves: they stay, so every later look would end in the
+// whole search as well.
+__host__ __device__ inline bool look_due(int iter, int blind, long long moved, long long ng) {
+  return iter > 1 && blind == 0 && 128 * moved <= ng;
+}
+__host__ __device__ inline bool look_few(long long listed, long long ns) {
+  return 16 * listed <= ns;
+}
+__host__ __device__ inline bool look_futile(long long stuck, long long ns) {
+  return !look_few(stuck, ns);
+}
+
 __host__ __device__ inline double det3(const double* w) {
   return w[0] * (w[3] * w[5] - w[4] * w[4]) - w[1] * (w[1] * w[5] - w[2] * w[4]) +
          w[2] * (w[1] * w[4] - w[2] * w[3]);

@@ -53,8 +53,10 @@ struct FrameDev {
   int iter;           // reference numIterEM (starts at 1)
   int active;         // keeps iterating
   int status;
+  unsigned long long again;  // queries the look found to search again, and (<< 32)
+                      // those of them it lists whatever moved
   int moved;          // means that moved since the last kNN search
-  int again;          // queries the look found to search again
+  int blind;          // a look listed too many whatever moved: no more looks
   int packed;         // every voxel's offset from its supervoxel's anchor is a
                       // small integer: the log-likelihood reads vpk (set to 1
                       // on the host, cleared by the moments kernel)

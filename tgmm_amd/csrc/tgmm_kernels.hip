@@ -419,6 +419,9 @@ __global__ void k_iter_init(DevPtrs P) {
                   ? 1
                   : 0;
   F->status = 0;
+  F->moved = 0;
+  F->again = 0;
+  F->blind = 0;
 }
 
 // Sum of alpha per frame before the first iteration (GMEM.cu:4167).
@@ -600,7 +603,11 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
   if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
   const FrameDev* F = P.fr + f;
   if (F->ncap == 0 || (need_active && !F->active)) return;  // empty slot / finished
-  if (which == 0 && threadIdx.x == 0) P.fr[f].moved = P.fr[f].again = 0;
+  if (which == 0 && threadIdx.x == 0) {
+    if (look_futile((long long)(F->again >> 32), F->ns)) P.fr[f].blind = 1;
+    P.fr[f].moved = 0;
+    P.fr[f].again = 0;
+  }
   const int* in;
   int* out;
   long long n;
@@ -917,10 +924,9 @@ __device__ inline float* knn_left(const DevPtrs& P, long long i) {
 // keeps is searched again.
 // In the EM's later iterations most means do not move at all in f32 (frame of
 // 60,000 Gaussians: 1% move in the 7th iteration, 0.1% in the 12th).
-__device__ inline bool knn_needed(const float* win, const int* qcell, const int* cell_mv,
+__device__ inline bool knn_needed(float kd, const int* qcell, const int* cell_mv,
                                   const float4* mv_pos, const float4* q4, const FrameDev* F,
                                   float s0, float s1, float s2, long long i) {
-  const float kd = win[2 * i];
   const int cell = qcell[i];
   if (!(kd >= 0.0f)) return true;
   const int nx = F->dims[0], ny = F->dims[1], nz = F->dims[2];
@@ -1290,18 +1296,20 @@ __device__ inline bool knn_wave(const DevPtrs& P, const KOpts& O, const FrameDev
 // which more than 1/128 of the frame's means moved. With a share p moved,
 // about 1 - (1 - p)^2K of the queries have to be searched again; by waves
 // that costs about five times a query of the lane search, so the line lies
-// where some tenth of the queries is left.
+// where some tenth of the queries is left (look_due).
 __device__ inline bool knn_looks(const FrameDev* F) {
-  return F->iter > 1 && 128LL * F->moved <= F->ng;
+  return look_due(F->iter, F->blind, F->moved, F->ng);
 }
 
 // After the look: whether the queries it listed are searched for by waves, or
 // the frame whole after all. The look cannot clear a query whose K-th
 // neighbour lies outside its block of cells, and with many slots or few means
-// a cell those are many, however few means moved (60,000 Gaussians, K = 8, 2
-// means a cell: 14.2 ms a solve by waves, 13.3 with this rule; 6 a cell: 10.7).
+// a cell those are many, however few means moved: where they alone are past
+// the line the frame's later iterations do not look (k_scan_frames, FrameDev's
+// blind). 60,000 Gaussians, K = 8, 2 means a cell: 13.3 ms a solve, 14.7 with
+// a look in every iteration that is due one, 13.8 with none (6 a cell: 11.0).
 __device__ inline bool knn_listed(const FrameDev* F) {
-  return knn_looks(F) && 16LL * F->again <= F->ns;
+  return knn_looks(F) && look_few((long long)(F->again & 0xffffffffull), F->ns);
 }
 
 // The look over every query, a lane each: those that may have other neighbours
@@ -1315,16 +1323,18 @@ __global__ __launch_bounds__(256) void k_knn_look(DevPtrs P, KOpts O) {
   if (f < 0 || !P.fr[f].active) return;
   const FrameDev* F = P.fr + f;
   if (!knn_looks(F)) return;
-  const bool need =
-      i < F->s0 + F->ns && knn_needed(knn_left(P, 0), P.qcell, P.cell_mv, P.mv_pos, P.q4, F,
-                                      O.scale[0], O.scale[1], O.scale[2], i);
-  const unsigned long long m = __ballot(need);
+  const bool in = i < F->s0 + F->ns;
+  const float kd = in ? *knn_left(P, i) : 0.0f;
+  const bool need = in && knn_needed(kd, P.qcell, P.cell_mv, P.mv_pos, P.q4, F, O.scale[0],
+                                     O.scale[1], O.scale[2], i);
+  const unsigned long long m = __ballot(need), stuck = __ballot(in && !(kd >= 0.0f));
   if (m == 0ull) return;
   const int lane = threadIdx.x & 63;
   int base = 0;
   if (lane == 0) {
     base = atomicAdd(P.knn_ctl + 3, __popcll(m));
-    atomicAdd(&P.fr[f].again, __popcll(m));
+    atomicAdd(&P.fr[f].again,
+              (unsigned long long)__popcll(m) | (unsigned long long)__popcll(stuck) << 32);
   }
   base = __builtin_amdgcn_readfirstlane(base);
   if (need) P.pairs[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)i;
@@ -1357,8 +1367,8 @@ __global__ __launch_bounds__(256) void k_knn_small(DevPtrs P, KOpts O) {
   if (f < 0 || !P.fr[f].active) return;
   const FrameDev* F = P.fr + f;
   if (i >= F->s0 + F->ns) return;  // whole waves
-  if (F->iter > 1 && !knn_needed(knn_left(P, 0), P.qcell, P.cell_mv, P.mv_pos, P.q4, F, O.scale[0],
-                                 O.scale[1], O.scale[2], i))
+  if (F->iter > 1 && !knn_needed(*knn_left(P, i), P.qcell, P.cell_mv, P.mv_pos, P.q4, F,
+                                 O.scale[0], O.scale[1], O.scale[2], i))
     return;
   const bool tie = knn_wave<KM>(P, O, F, i, rows[w]);
   if (tie && (threadIdx.x & 63) == 0)
