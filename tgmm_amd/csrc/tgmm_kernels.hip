@@ -2503,8 +2503,12 @@ __global__ __launch_bounds__(256) void k_pair_scatter(DevPtrs P, KOpts O) {
 // one at a time, among those with more than kSortShort pairs (listed by the
 // pair scan): up to kRunLds runs ranked in LDS, a run a thread; beyond, the
 // pairs laid out and sorted in LDS (bitonic), or, past kSortLds pairs, the
-// runs ranked from memory. Both sides read the run count; whichever handles a
-// Gaussian clears it (the other, reading 0, writes nothing).
+// runs ranked against all of them, kRunTile at a time through LDS, eight a
+// thread (four lists of 20,000 single-pair runs: 8 ms an iteration; with each
+// comparison's code and length read from memory 103, with only the codes of
+// the pairs 96).
+// Both sides read the run count; whichever handles a Gaussian clears it (the
+// other, reading 0, writes nothing).
 // Latency-bound. Against sorting the pairs themselves: 60,000 Gaussians 22.4
 // -> 12.5 us, 200 Gaussians 5.1 -> 3.6 us, per-voxel frames of 4.9M and 40,000
 // voxels 156 -> 49.5 and 19.5 -> 9.5 us.
@@ -2513,6 +2517,7 @@ __global__ __launch_bounds__(256) void k_pair_scatter(DevPtrs P, KOpts O) {
 // list is a chain of barriers and LDS round trips (about 20 us for 512 pairs),
 // and lists of scattered voxels have as many runs as pairs.
 constexpr int kRunLds = 512;
+constexpr int kRunTile = kSortLds / 2;
 constexpr int kSortLongFew = 64;
 constexpr int kSortLongMany = 2048;
 inline int sort_long_blocks(const DevPtrs& P) {
@@ -2622,13 +2627,38 @@ __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int n
       continue;
     }
     if (L > kSortLds) {
-      for (int r = t; r < nr; r += 256) {
-        const int c = P.pairs[st + r], n = P.run_len[st + r];
-        int at = 0;
-        for (int i = 0; i < nr; i++) at += P.pairs[st + i] < c ? P.run_len[st + i] : 0;
-        for (int u = 0; u < n; u++) P.pairs_sorted[st + at + u] = c + (u << kPairShift);
+      constexpr int R = 8;  // runs a thread ranks at once
+      int2* tile = reinterpret_cast<int2*>(sh);
+      for (int r0 = 0; r0 < nr; r0 += 256 * R) {
+        int c[R], at[R];
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+          const int r = r0 + t + 256 * q;
+          c[q] = r < nr ? P.pairs[st + r] : INT_MIN;
+          at[q] = 0;
+        }
+        for (int b = 0; b < nr; b += kRunTile) {
+          const int m = min(kRunTile, nr - b);
+          __syncthreads();  // the tile before has been read
+          for (int i = t; i < m; i += 256)
+            tile[i] = make_int2(P.pairs[st + b + i], P.run_len[st + b + i]);
+          __syncthreads();
+#pragma unroll 4
+          for (int i = 0; i < m; i++) {
+            const int2 v = tile[i];
+#pragma unroll
+            for (int q = 0; q < R; q++) at[q] += v.x < c[q] ? v.y : 0;
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+          const int r = r0 + t + 256 * q;
+          if (r >= nr) continue;
+          const int n = P.run_len[st + r];
+          for (int u = 0; u < n; u++) P.pairs_sorted[st + at[q] + u] = c[q] + (u << kPairShift);
+        }
       }
-      __syncthreads();  // every thread has read the count
+      __syncthreads();  // every thread has read the count, and sh is free
       if (t == 0) P.run_cnt[k] = 0;
       continue;
     }
@@ -2672,7 +2702,7 @@ __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int n
 }
 
 __global__ __launch_bounds__(256) void k_seg_sort(DevPtrs P, int nshort, int nlong) {
-  __shared__ int sh[kSortLds > 32 * kSortShort ? kSortLds : 32 * kSortShort];
+  __shared__ __align__(16) int sh[kSortLds > 32 * kSortShort ? kSortLds : 32 * kSortShort];
   if ((int)blockIdx.x < nshort)
     seg_sort_short(P, sh);
   else
