@@ -1342,8 +1342,11 @@ __global__ __launch_bounds__(256) void k_knn_look(DevPtrs P, KOpts O) {
 
 // The lane search of every query, blockDim.x / QL a block.
 // VALU-bound: 5.7k instructions a wave at K = 8 (60,000 Gaussians: 152 us).
+// Four waves a SIMD, three for K > 8 (168 registers: left to itself the
+// compiler takes 170 for several lanes a query and a wave less fits; 10,000
+// Gaussians, K = 16, a solve with 2 lanes 2.70 -> 2.45 ms, 4 lanes 3.16 -> 2.79).
 template <int KM, int KC, int QL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KM <= 8 ? 4 : 1))) void k_knn(DevPtrs P, KOpts O) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KM <= 8 ? 4 : 3))) void k_knn(DevPtrs P, KOpts O) {
   extern __shared__ float2 kq[];
   const long long qpb = blockDim.x / QL;  // queries per block
   const long long i = (long long)blockIdx.x * qpb + threadIdx.x / QL;
