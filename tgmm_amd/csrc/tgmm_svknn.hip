@@ -27,10 +27,13 @@
 //     the start (a superset of the ones the scan inserts, since the threshold
 //     only falls) and walks its marks in order with the exact test.
 // Thresholds only fall, so a stale one only keeps more.
-// With a coordinate that is not finite (or beyond 1e18) anywhere a distance
-// can be NaN, and a NaN threshold takes any next reference: the kernel then
-// walks every reference with the reference's own test and slot update
-// (scan_all).
+// With a coordinate that is not finite (or beyond 1e18) a distance can be NaN,
+// and a NaN threshold takes any next reference: a wave with such a query, and
+// every wave if a reference is such, walks the references with the
+// reference's own test and slot update (scan_all). It leaves out a block of
+// 64 that is farther from each of its queries than the query's threshold; a
+// block that holds such a reference has an unbounded box and is always taken,
+// as every block is for such a query.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -54,7 +57,7 @@ constexpr int kMaxPacked = 1 << 27;  // reference indices that fit beside a slot
 
 // Written by the preparation kernels, cleared before: the largest ordered
 // image of the query coordinates (hi) and of their complements (lo) per axis,
-// and whether a coordinate is not finite.
+// and whether a reference's coordinate is not regular.
 struct KnnPrep {
   unsigned hi[3], lo[3];
   unsigned irregular;
@@ -72,7 +75,8 @@ __device__ inline float unordered(unsigned u) {
 __device__ inline bool regular(float v) { return fabsf(v) <= 1e18f; }
 
 // Bounding box of each block of 64 references (box[a][b] = min, box[3+a][b]
-// = max of coordinate a), and, in the blocks after, the queries' extent.
+// = max of coordinate a; unbounded with an irregular coordinate), and, in the
+// blocks after, the queries' extent.
 __global__ __launch_bounds__(kKB) void k_svknn_boxes(const float* __restrict__ ref, int R,
                                                      int Rp, int nblk, float* __restrict__ box,
                                                      const float* __restrict__ query, long long Q,
@@ -100,8 +104,6 @@ __global__ __launch_bounds__(kKB) void k_svknn_boxes(const float* __restrict__ r
         if (regular(v)) {
           lo[a] = fminf(lo[a], v);
           hi[a] = fmaxf(hi[a], v);
-        } else {
-          bad = true;
         }
       }
   }
@@ -110,12 +112,13 @@ __global__ __launch_bounds__(kKB) void k_svknn_boxes(const float* __restrict__ r
       lo[a] = fminf(lo[a], __shfl_xor(lo[a], m, 64));
       hi[a] = fmaxf(hi[a], __shfl_xor(hi[a], m, 64));
     }
-  if (__any(bad) && threadIdx.x == 0) atomicOr(&prep->irregular, 1u);
+  bad = __any(bad);
   if (threadIdx.x != 0) return;
+  if (bad) atomicOr(&prep->irregular, 1u);
   for (int a = 0; a < 3; a++) {
     if (b < nblk) {
-      box[(long long)a * nblk + b] = lo[a];
-      box[(long long)(3 + a) * nblk + b] = hi[a];
+      box[(long long)a * nblk + b] = bad ? -INFINITY : lo[a];
+      box[(long long)(3 + a) * nblk + b] = bad ? INFINITY : hi[a];
     } else if (lo[a] <= hi[a]) {
       atomicMax(&prep->hi[a], ordered(hi[a]));
       atomicMax(&prep->lo[a], ~ordered(lo[a]));
@@ -279,13 +282,23 @@ __device__ inline unsigned dpp_or(unsigned v) {  // OR over the group
   return v;
 }
 
-// The reference's scan over every reference (any coordinates) for the query
-// of a group of QL lanes, which split the marking of each 64.
-__device__ __noinline__ void scan_all(float q0, float q1, float q2, bool live, long long q,
-                                      long long Q, const float* __restrict__ ref, int R, int Rp,
-                                      int K, float s0, float s1, float s2, int* __restrict__ ind,
-                                      float* __restrict__ dist) {
-  const int sub = threadIdx.x % QL;
+// The reference's scan (any coordinates) for query q4[i] of a group of L lanes,
+// which split the marking of each 64.
+template <int L>
+__device__ __noinline__ void scan_all(const float4* __restrict__ q4, long long i, long long Q,
+                                      const float* __restrict__ ref, int R, int Rp, int K,
+                                      float s0, float s1, float s2,
+                                      const float* __restrict__ box, int nblk,
+                                      int* __restrict__ ind, float* __restrict__ dist) {
+  const int sub = threadIdx.x % L;
+  const bool live = i < Q;
+  const float4 qq = live ? q4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  const float q0 = qq.x, q1 = qq.y, q2 = qq.z;
+  const long long q = __float_as_int(qq.w);
+  // only a regular query's distances to a block's regular references are
+  // bounded by its box
+  const bool all = !(regular(q0) && regular(q1) && regular(q2) && regular(s0) && regular(s1) &&
+                     regular(s2));
   float md[kKM];
   int mi[kKM];
 #pragma unroll
@@ -295,22 +308,32 @@ __device__ __noinline__ void scan_all(float q0, float q1, float q2, bool live, l
   }
   float thr = live ? 1e32f : -INFINITY;  // a lane past the end inserts nothing
   int pos = 0;
-  for (int rb = 0; rb < R; rb += 64) {
+  for (int b = 0; b < nblk; b++) {
+    const float lb = gap_bound(fmaxf(box[b] - q0, q0 - box[3 * nblk + b]),
+                               fmaxf(box[nblk + b] - q1, q1 - box[4 * nblk + b]),
+                               fmaxf(box[2 * nblk + b] - q2, q2 - box[5 * nblk + b]), s0, s1, s2);
+    if (!__any(all || !(lb > thr))) continue;  // no query of the wave takes any of it
+    const int rb = b * kKB;
     const float t0 = thr;
     unsigned cl = 0u, ch = 0u;
 #pragma unroll
-    for (int v = 0; v < 64 / QL; v++) {
-      const int r = rb + v * QL + sub;  // below Rp
+    for (int v = 0; v < 64 / L; v++) {
+      const int r = rb + v * L + sub;  // below Rp
       const float d =
           svdist(q0, q1, q2, make_float4(ref[r], ref[r + Rp], ref[r + 2 * Rp], 0.0f), s0, s1, s2);
-      const unsigned bit = (d > t0) ? 0u : 1u << ((v * QL + sub) & 31);
-      if (v * QL < 32)
+      const unsigned bit = (d > t0) ? 0u : 1u << ((v * L + sub) & 31);
+      if (v * L < 32)
         cl |= bit;
       else
         ch |= bit;
     }
+    if constexpr (L > 1) {
+      static_assert(L == QL, "one group size for the lane exchanges");
+      cl = dpp_or(cl);
+      ch = dpp_or(ch);
+    }
     const unsigned long long nmask = R - rb < 64 ? (1ull << (R - rb)) - 1ull : ~0ull;
-    unsigned long long cand = (((unsigned long long)dpp_or(ch) << 32) | dpp_or(cl)) & nmask;
+    unsigned long long cand = (((unsigned long long)ch << 32) | cl) & nmask;
     while (cand) {
       const int u = __builtin_ctzll(cand), r = rb + u;
       cand &= cand - 1ull;
@@ -341,10 +364,34 @@ __device__ __noinline__ void scan_all(float q0, float q1, float q2, bool live, l
   if (!live) return;
 #pragma unroll
   for (int j = 0; j < kKM; j++)
-    if (j < K && j % QL == sub) {
+    if (j < K && j % L == sub) {
       ind[q + j * Q] = mi[j];
       if (dist) dist[q + j * Q] = md[j];
     }
+}
+
+// Whether a distance to some reference may not be bounded by the boxes, or the
+// references are too many to be packed: then every query is scanned for by
+// scan_all, from kScanAlone queries on in a kernel of its own with a lane a
+// query. Four lanes shorten the marking, one does more queries a wave of the
+// walk over the marks, which is most of it, where there are 64-query waves for
+// every SIMD: K = 10, one reference NaN / 1% of them, four lanes and one,
+// 5,000 queries and references 0.76 / 1.03 and 0.86 / 1.15 ms a call, 100,000
+// 7.7 / 26.9 and 6.95 / 15.9 (4.2 where all are regular). Beside the other
+// form in one kernel its registers (64 references' loads together) cost that a
+// tenth.
+constexpr long long kScanAlone = 65536;
+__device__ inline bool scans_all(const KnnPrep* prep, int R, float s0, float s1, float s2) {
+  return prep->irregular != 0 || !regular(s0) || !regular(s1) || !regular(s2) || R >= kMaxPacked;
+}
+
+__global__ __launch_bounds__(64) void k_svknn_all(
+    const float4* __restrict__ q4, long long Q, const float* __restrict__ ref, int R, int Rp,
+    int K, float s0, float s1, float s2, const float* __restrict__ box, int nblk,
+    const KnnPrep* __restrict__ prep, int* __restrict__ ind, float* __restrict__ dist) {
+  if (scans_all(prep, R, s0, s1, s2))
+    scan_all<1>(q4, (long long)blockIdx.x * 64 + threadIdx.x, Q, ref, R, Rp, K, s0, s1, s2, box,
+                nblk, ind, dist);
 }
 
 // QL lanes share a query. ref is SoA with axis stride Rp = nblk * 64 (padded
@@ -378,8 +425,10 @@ __global__ __launch_bounds__(64) void k_svknn(
   const float4 qq = live ? q4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   const float q0 = qq.x, q1 = qq.y, q2 = qq.z;
   const long long q = __float_as_int(qq.w);
-  if (prep->irregular != 0 || !regular(s0) || !regular(s1) || !regular(s2) || R >= kMaxPacked) {
-    scan_all(q0, q1, q2, live, q, Q, ref, R, Rp, K, s0, s1, s2, ind, dist);
+  const bool every = scans_all(prep, R, s0, s1, s2);
+  if (every && Q >= kScanAlone) return;
+  if (every || __any(!regular(q0) || !regular(q1) || !regular(q2))) {
+    scan_all<QL>(q4, i, Q, ref, R, Rp, K, s0, s1, s2, box, nblk, ind, dist);
     return;
   }
   // the box around the wave's queries
@@ -623,6 +672,10 @@ extern "C" int tgmm_knnCUDA_(int* ind, float* dist, const float* query, const fl
   k_svknn<<<(unsigned)((Q * QL + 63) / 64), 64, 0, 0>>>(dq4, Q, dr, (int)R, (int)Rp, KNN, s0, s1,
                                                         s2, dbox, nblk, dprep, dind,
                                                         dist ? ddist : nullptr);
+  if (Q >= kScanAlone)  // returns at once unless it has to
+    k_svknn_all<<<(unsigned)((Q + 63) / 64), 64, 0, 0>>>(dq4, Q, dr, (int)R, (int)Rp, KNN, s0, s1,
+                                                         s2, dbox, nblk, dprep, dind,
+                                                         dist ? ddist : nullptr);
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "kernel launch");
   if ((e = hipMemcpy(ind, dind, (size_t)Q * KNN * 4, hipMemcpyDeviceToHost)) != hipSuccess ||
       (dist && (e = hipMemcpy(dist, ddist, (size_t)Q * KNN * 4, hipMemcpyDeviceToHost)) !=
