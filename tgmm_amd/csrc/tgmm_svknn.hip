@@ -146,13 +146,14 @@ __device__ inline int query_cell(const KnnPrep* prep, float x, float y, float z,
   return c;
 }
 
-__global__ __launch_bounds__(256) void k_svknn_count(const float* __restrict__ query, long long Q,
-                                                     float s0, float s1, float s2,
+// (the n queries of one piece; axes Q apart)
+__global__ __launch_bounds__(256) void k_svknn_count(const float* __restrict__ query, long long n,
+                                                     long long Q, float s0, float s1, float s2,
                                                      const KnnPrep* __restrict__ prep,
                                                      int* __restrict__ cell,
                                                      int* __restrict__ cnt) {
   const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (q >= Q) return;
+  if (q >= n) return;
   const int c = query_cell(prep, query[q], query[q + Q], query[q + 2 * Q], s0, s1, s2);
   cell[q] = c;
   atomicAdd(cnt + c, 1);
@@ -193,11 +194,12 @@ __global__ __launch_bounds__(1024) void k_svknn_scan(int* __restrict__ cnt) {
 }
 
 __global__ __launch_bounds__(256) void k_svknn_scatter(const float* __restrict__ query,
-                                                       long long Q, const int* __restrict__ cell,
+                                                       long long n, long long Q,
+                                                       const int* __restrict__ cell,
                                                        int* __restrict__ start,
                                                        float4* __restrict__ q4) {
   const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (q >= Q) return;
+  if (q >= n) return;
   q4[atomicAdd(start + cell[q], 1)] =
       make_float4(query[q], query[q + Q], query[q + 2 * Q], __int_as_float((int)q));
 }
@@ -285,13 +287,14 @@ __device__ inline unsigned dpp_or(unsigned v) {  // OR over the group
 // The reference's scan (any coordinates) for query q4[i] of a group of L lanes,
 // which split the marking of each 64.
 template <int L>
-__device__ __noinline__ void scan_all(const float4* __restrict__ q4, long long i, long long Q,
-                                      const float* __restrict__ ref, int R, int Rp, int K,
+__device__ __noinline__ void scan_all(const float4* __restrict__ q4, long long i, long long n,
+                                      long long Q, const float* __restrict__ ref, int R, int Rp,
+                                      int K,
                                       float s0, float s1, float s2,
                                       const float* __restrict__ box, int nblk,
                                       int* __restrict__ ind, float* __restrict__ dist) {
   const int sub = threadIdx.x % L;
-  const bool live = i < Q;
+  const bool live = i < n;
   const float4 qq = live ? q4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   const float q0 = qq.x, q1 = qq.y, q2 = qq.z;
   const long long q = __float_as_int(qq.w);
@@ -386,11 +389,11 @@ __device__ inline bool scans_all(const KnnPrep* prep, int R, float s0, float s1,
 }
 
 __global__ __launch_bounds__(64) void k_svknn_all(
-    const float4* __restrict__ q4, long long Q, const float* __restrict__ ref, int R, int Rp,
-    int K, float s0, float s1, float s2, const float* __restrict__ box, int nblk,
+    const float4* __restrict__ q4, long long n, long long Q, const float* __restrict__ ref, int R,
+    int Rp, int K, float s0, float s1, float s2, const float* __restrict__ box, int nblk,
     const KnnPrep* __restrict__ prep, int* __restrict__ ind, float* __restrict__ dist) {
   if (scans_all(prep, R, s0, s1, s2))
-    scan_all<1>(q4, (long long)blockIdx.x * 64 + threadIdx.x, Q, ref, R, Rp, K, s0, s1, s2, box,
+    scan_all<1>(q4, (long long)blockIdx.x * 64 + threadIdx.x, n, Q, ref, R, Rp, K, s0, s1, s2, box,
                 nblk, ind, dist);
 }
 
@@ -412,8 +415,8 @@ __global__ __launch_bounds__(64) void k_svknn_all(
 // query over blocks of 64 references skipped by their boxes alone; 5,208
 // queries, 0.23 ms against 0.91.
 __global__ __launch_bounds__(64) void k_svknn(
-    const float4* __restrict__ q4, long long Q, const float* __restrict__ ref, int R, int Rp,
-    int K, float s0, float s1, float s2, const float* __restrict__ box, int nblk,
+    const float4* __restrict__ q4, long long n, long long Q, const float* __restrict__ ref, int R,
+    int Rp, int K, float s0, float s1, float s2, const float* __restrict__ box, int nblk,
     const KnnPrep* __restrict__ prep, int* __restrict__ ind, float* __restrict__ dist) {
 #pragma clang fp contract(off)
   constexpr int E = 12 / QL;  // places per lane
@@ -421,14 +424,14 @@ __global__ __launch_bounds__(64) void k_svknn(
   __shared__ float4 buf[64 + 64 * kKU];
   const int lane = threadIdx.x, sub = lane % QL;
   const long long i = (long long)blockIdx.x * (64 / QL) + lane / QL;
-  const bool live = i < Q;
+  const bool live = i < n;
   const float4 qq = live ? q4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   const float q0 = qq.x, q1 = qq.y, q2 = qq.z;
   const long long q = __float_as_int(qq.w);
   const bool every = scans_all(prep, R, s0, s1, s2);
-  if (every && Q >= kScanAlone) return;
+  if (every && n >= kScanAlone) return;
   if (every || __any(!regular(q0) || !regular(q1) || !regular(q2))) {
-    scan_all<QL>(q4, i, Q, ref, R, Rp, K, s0, s1, s2, box, nblk, ind, dist);
+    scan_all<QL>(q4, i, n, Q, ref, R, Rp, K, s0, s1, s2, box, nblk, ind, dist);
     return;
   }
   // the box around the wave's queries
@@ -453,8 +456,8 @@ __global__ __launch_bounds__(64) void k_svknn(
   float thr = live ? 1e32f : -INFINITY;  // the last place
   float second = K > 1 ? thr : -INFINITY;  // the place before
   int tail = dpp_last(pay[E - 1]);
-  // n collected references at buf[base ..] through the scan
-  auto process = [&](int base, int n) {
+  // cnt collected references at buf[base ..] through the scan
+  auto process = [&](int base, int cnt) {
     unsigned cl = 0u, ch = 0u;
     const float t0 = thr;
 #pragma unroll
@@ -470,7 +473,7 @@ __global__ __launch_bounds__(64) void k_svknn(
     cl = dpp_or(cl);
     ch = dpp_or(ch);
     unsigned long long cand = ((unsigned long long)ch << 32) | cl;
-    cand &= n < 64 ? (1ull << n) - 1ull : ~0ull;
+    cand &= cnt < 64 ? (1ull << cnt) - 1ull : ~0ull;
     while (cand) {  // the same in the group's lanes
       const int u = __builtin_ctzll(cand);
       cand &= cand - 1ull;
@@ -579,6 +582,12 @@ __global__ __launch_bounds__(64) void k_svknn(
     }
 }
 
+// Queries sorted and searched for together: four lanes each and a 32-bit index
+// within the piece, for any number of queries (2^30 at once would be a grid of
+// 2^32 threads, which no launch takes), and 20 bytes of scratch for no more
+// than a piece of them.
+constexpr long long kPiece = 1LL << 22;
+
 inline size_t up256(size_t n) { return (n + 255) & ~size_t(255); }
 
 struct KnnWs {
@@ -621,14 +630,15 @@ extern "C" int tgmm_knnCUDA_(int* ind, float* dist, const float* query, const fl
   const long long Q = query_nb, R = ref_nb;
   const int nblk = (int)((R + kKB - 1) / kKB);
   const long long Rp = (long long)nblk * kKB;
+  const long long piece = std::min(Q, kPiece);
   const size_t o_q = 0;
   const size_t o_r = o_q + up256((size_t)Q * 12);
   const size_t o_box = o_r + up256((size_t)Rp * 12);
   const size_t o_prep = o_box + up256((size_t)nblk * 24);
   const size_t o_cnt = o_prep + 256;
   const size_t o_cell = o_cnt + up256((size_t)kCells * 4);
-  const size_t o_q4 = o_cell + up256((size_t)Q * 4);
-  const size_t o_ind = o_q4 + up256((size_t)Q * 16);
+  const size_t o_q4 = o_cell + up256((size_t)piece * 4);
+  const size_t o_ind = o_q4 + up256((size_t)piece * 16);
   const size_t o_dist = o_ind + up256((size_t)Q * KNN * 4);
   const size_t total = o_dist + up256((size_t)Q * KNN * 4);
   std::lock_guard<std::mutex> lk(g_mu);
@@ -663,19 +673,24 @@ extern "C" int tgmm_knnCUDA_(int* ind, float* dist, const float* query, const fl
   if ((e = hipMemsetAsync(dprep, 0, o_cell - o_prep, 0)) != hipSuccess)
     return hip_fail(e, "clearing the counts");
   const float s0 = scale[0], s1 = scale[1], s2 = scale[2];
-  const unsigned qb = (unsigned)((Q + 255) / 256);
   k_svknn_boxes<<<nblk + (unsigned)std::min<long long>(256, (Q + kKB - 1) / kKB), kKB, 0, 0>>>(
       dr, (int)R, (int)Rp, nblk, dbox, dq, Q, dprep);
-  k_svknn_count<<<qb, 256, 0, 0>>>(dq, Q, s0, s1, s2, dprep, dcell, dcnt);
-  k_svknn_scan<<<1, 1024, 0, 0>>>(dcnt);
-  k_svknn_scatter<<<qb, 256, 0, 0>>>(dq, Q, dcell, dcnt, dq4);
-  k_svknn<<<(unsigned)((Q * QL + 63) / 64), 64, 0, 0>>>(dq4, Q, dr, (int)R, (int)Rp, KNN, s0, s1,
-                                                        s2, dbox, nblk, dprep, dind,
-                                                        dist ? ddist : nullptr);
-  if (Q >= kScanAlone)  // returns at once unless it has to
-    k_svknn_all<<<(unsigned)((Q + 63) / 64), 64, 0, 0>>>(dq4, Q, dr, (int)R, (int)Rp, KNN, s0, s1,
-                                                         s2, dbox, nblk, dprep, dind,
-                                                         dist ? ddist : nullptr);
+  for (long long p = 0; p < Q; p += piece) {
+    const long long n = std::min(piece, Q - p);
+    const unsigned qb = (unsigned)((n + 255) / 256);
+    int* pind = dind + p;
+    float* pdist = dist ? ddist + p : nullptr;
+    if (p > 0 && (e = hipMemsetAsync(dcnt, 0, (size_t)kCells * 4, 0)) != hipSuccess)
+      return hip_fail(e, "clearing the counts");
+    k_svknn_count<<<qb, 256, 0, 0>>>(dq + p, n, Q, s0, s1, s2, dprep, dcell, dcnt);
+    k_svknn_scan<<<1, 1024, 0, 0>>>(dcnt);
+    k_svknn_scatter<<<qb, 256, 0, 0>>>(dq + p, n, Q, dcell, dcnt, dq4);
+    k_svknn<<<(unsigned)((n * QL + 63) / 64), 64, 0, 0>>>(dq4, n, Q, dr, (int)R, (int)Rp, KNN, s0,
+                                                          s1, s2, dbox, nblk, dprep, pind, pdist);
+    if (n >= kScanAlone)  // returns at once unless it has to
+      k_svknn_all<<<(unsigned)((n + 63) / 64), 64, 0, 0>>>(dq4, n, Q, dr, (int)R, (int)Rp, KNN, s0,
+                                                           s1, s2, dbox, nblk, dprep, pind, pdist);
+  }
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "kernel launch");
   if ((e = hipMemcpy(ind, dind, (size_t)Q * KNN * 4, hipMemcpyDeviceToHost)) != hipSuccess ||
       (dist && (e = hipMemcpy(dist, ddist, (size_t)Q * KNN * 4, hipMemcpyDeviceToHost)) !=
