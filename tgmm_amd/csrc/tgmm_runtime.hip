@@ -54,33 +54,16 @@ extern "C" int tgmm_device_count(int* count) {
 // -------------------------------------------------------------- workspace --
 static long long round_up(long long x, long long a) { return ((x + a - 1) / a) * a; }
 
-int ws_alloc(Workspace* w, const WsShape& sh, int K) {
-  w->sh = sh;
-  w->K = K;
+// Every array of a workspace, in allocation order: each(&pointer, bytes)
+// returns TGMM_OK to go on. What a workspace takes is counted from this list
+// too (ws_bytes), so the two cannot differ.
+template <class Each>
+static int ws_arrays(Workspace* w, const WsShape& sh, int K, Each each) {
   DevPtrs& P = w->P;
-  std::memset(&P, 0, sizeof(P));
-  P.Scap = sh.Scap;
-  P.Gcap = sh.Gcap;
-  P.Ccap = sh.Ccap;
-  P.Sext = sh.Scap;
-  P.Gext = sh.Gcap;
-  P.Cext = sh.Ccap;
-  P.Vcap = sh.Vcap;
-  P.Fcap = sh.Fcap;
-  auto A = [&](void** p, size_t bytes) -> int {
-    bytes = std::max<size_t>(bytes, 256);
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) {
-      tgmm_set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
-      return TGMM_ERR_OOM;
-    }
-    w->allocs.push_back(*p);
-    w->bytes += bytes;
-    return TGMM_OK;
-  };
-#define AL(ptr, n) \
-  if (int rc_ = A((void**)&(ptr), (size_t)(n) * sizeof(*(ptr)))) return rc_
   const long long S = sh.Scap, G = sh.Gcap, C = sh.Ccap, V = sh.Vcap, F = sh.Fcap;
+#define AL(ptr, n)                                                                   \
+  if (int rc_ = each((void**)&(ptr), std::max<size_t>((size_t)(n) * sizeof(*(ptr)), 256))) \
+  return rc_
   AL(P.vx, V);
   AL(P.vy, V);
   AL(P.vz, V);
@@ -139,18 +122,45 @@ int ws_alloc(Workspace* w, const WsShape& sh, int K) {
   return TGMM_OK;
 }
 
+int ws_alloc(Workspace* w, const WsShape& sh, int K) {
+  w->sh = sh;
+  w->K = K;
+  DevPtrs& P = w->P;
+  std::memset(&P, 0, sizeof(P));
+  P.Scap = sh.Scap;
+  P.Gcap = sh.Gcap;
+  P.Ccap = sh.Ccap;
+  P.Sext = sh.Scap;
+  P.Gext = sh.Gcap;
+  P.Cext = sh.Ccap;
+  P.Vcap = sh.Vcap;
+  P.Fcap = sh.Fcap;
+  return ws_arrays(w, sh, K, [w](void** p, size_t bytes) -> int {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+      tgmm_set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+      return TGMM_ERR_OOM;
+    }
+    w->allocs.push_back(*p);
+    w->bytes += bytes;
+    return TGMM_OK;
+  });
+}
+
 void ws_free(Workspace* w) {
   for (void* p : w->allocs) (void)hipFree(p);
   w->allocs.clear();
   w->bytes = 0;
 }
 
-long long ws_bytes_estimate(const WsShape& sh, int K) {
-  const long long S = sh.Scap, G = sh.Gcap, C = sh.Ccap, V = sh.Vcap;
-  return 24 * V + S * (16 + 8 + 4 + 12 + 80 + 80 + 12 + 16 + 16LL * K + 1 + 4 + 8) +
-         G * (4 + 8 * GS_NFIELDS * 2 + 1 + 96 + 8 + 64 + 12 + 4 + 8 + 12 + 4 + 1 + 16 + 288 +
-              68 + 4) +
-         8 * C + 64 * sh.Fcap;
+long long ws_bytes(const WsShape& sh, int K) {
+  Workspace w;
+  long long total = 0;
+  ws_arrays(&w, sh, K, [&total](void**, size_t bytes) -> int {
+    total += (long long)bytes;
+    return TGMM_OK;
+  });
+  return total;
 }
 
 // ------------------------------------------------------------------ batch --

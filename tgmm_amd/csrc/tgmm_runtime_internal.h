@@ -65,7 +65,9 @@ struct tgmm_batch {
 void tgmm_set_error(const char* fmt, ...);
 int ws_alloc(Workspace* w, const WsShape& sh, int K);
 void ws_free(Workspace* w);
-long long ws_bytes_estimate(const WsShape& sh, int K);
+long long ws_bytes(const WsShape& sh, int K);  // what ws_alloc allocates
+// The workspace of a server with max_frames slots and a budget of device memory.
+WsShape server_shape(long long budget, int max_frames, int K);
 tgmm::KOpts make_kopts(const tgmm_em_opts& o, const float* scale_reg);
 void records_to_soa(const GaussianMixtureModelCUDA* gm, long long G, long long g0, long long Gcap,
                     double* gs, unsigned char* fixed, int* svkeep);

@@ -250,6 +250,27 @@ static int server_capture(tgmm_server* s) {
   return TGMM_OK;
 }
 
+// Capacity from the budget: supervoxels >= 8 voxels and Gaussians >= 32 voxels
+// on average, two grid cells per Gaussian plus slack per slot. A power of two
+// of voxels, at least 2^20; where the last doubling is up to a sixteenth above
+// the budget, it is taken and trimmed to fit instead of left out.
+WsShape server_shape(long long budget, int max_frames, int K) {
+  auto shape = [&](long long V) {
+    WsShape t;
+    t.Fcap = max_frames;
+    t.Vcap = V;
+    t.Scap = rup(V / 8 + 256LL * t.Fcap, kAlign);
+    t.Gcap = rup(V / 32 + 256LL * t.Fcap, kAlign);
+    t.Ccap = rup(t.Gcap / 2 + 2LL * kCB * t.Fcap, kCB);
+    return t;
+  };
+  constexpr long long kLeast = 1LL << 20;
+  long long V = kLeast;
+  while (2 * V <= (1LL << 31) && ws_bytes(shape(2 * V), K) - budget / 16 <= budget) V *= 2;
+  for (const long long step = V / 128; V > kLeast && ws_bytes(shape(V), K) > budget;) V -= step;
+  return shape(V);
+}
+
 extern "C" int tgmm_server_create(int device, const tgmm_server_opts* opts, tgmm_server** out) {
   if (!opts || !out || opts->max_frames_in_flight < 1 || opts->hbm_budget_bytes <= 0) {
     tgmm_set_error("tgmm_server_create: bad arguments");
@@ -269,26 +290,7 @@ extern "C" int tgmm_server_create(int device, const tgmm_server_opts* opts, tgmm
   s->device = device;
   s->o = *opts;
   s->ko = make_kopts(e, nullptr);
-  // capacity from the budget: supervoxels >= 8 voxels and Gaussians >= 32
-  // voxels on average, two grid cells per Gaussian plus slack per slot
-  WsShape sh;
-  sh.Fcap = opts->max_frames_in_flight;
-  long long V = 1 << 20;
-  for (;;) {
-    WsShape t;
-    t.Fcap = sh.Fcap;
-    const long long V2 = V * 2;
-    t.Vcap = V2;
-    t.Scap = rup(V2 / 8 + 256LL * t.Fcap, kAlign);
-    t.Gcap = rup(V2 / 32 + 256LL * t.Fcap, kAlign);
-    t.Ccap = rup(t.Gcap / 2 + 2LL * kCB * t.Fcap, kCB);
-    if (ws_bytes_estimate(t, e.K) > opts->hbm_budget_bytes || V2 > (1LL << 31)) break;
-    V = V2;
-  }
-  sh.Vcap = V;
-  sh.Scap = rup(V / 8 + 256LL * sh.Fcap, kAlign);
-  sh.Gcap = rup(V / 32 + 256LL * sh.Fcap, kAlign);
-  sh.Ccap = rup(sh.Gcap / 2 + 2LL * kCB * sh.Fcap, kCB);
+  const WsShape sh = server_shape(opts->hbm_budget_bytes, opts->max_frames_in_flight, e.K);
   if (int rc = ws_alloc(&s->ws, sh, e.K)) {
     ws_free(&s->ws);
     delete s;
