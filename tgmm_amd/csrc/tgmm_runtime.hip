@@ -214,18 +214,26 @@ KOpts make_kopts(const tgmm_em_opts& o, const float* scale_reg) {
   return k;
 }
 
-// Each line lies where the measured times of the two sides cross (us):
+// Each line lies between the measured sizes where the two sides cross (kernel
+// times in us, but solves of 12 iterations in ms for the kNN search). S and G
+// are what the frames hold, without the padding of their ranges: 32 frames of
+// 20 Gaussians have lists of 11.5 pairs and, padded, seem to have 1 (4 lanes
+// 11.4, 8 lanes 8.8).
 //   M-step lanes 4 / 8 / 16 by the mean pair list S / G: 1.7 pairs 20 / 34 /
-//     46 (153,000 Gaussians), 4.2 pairs 8.4 / 9.6 / 10.7 (200), 10.6 pairs 15.4
-//     / 11.0 / 12.5 (10,000), 11.1 pairs 34 / 26.5 / 28.8 (60,000), 485 pairs
-//     (per-voxel, 10,000) 98 / 65 / 49;
+//     46 (153,000 Gaussians), 4.4 pairs 10.7 / 10.2 / 12.3 (10,000), 6.4 pairs
+//     9.3 / 10.9 / 11.7 (300), 9.8 / 10.1 / 11.6 (2,000) and 12.3 / 10.5 / 12.4
+//     (10,000), 25 pairs 11.5 / 12.5, 13.8 / 13.2 and 14.9 / 15.1 with 8 / 16,
+//     40 pairs 13.5 / 13.5, 16.7 / 15.7 and 18.6 / 17.3, 485 pairs (per-voxel)
+//     65 / 49;
 //   log-likelihood in blocks of 16 supervoxels, two voxels a thread, against
 //     32 and four, where there are blocks to fill the chip: 128 / 140 (668,000
 //     supervoxels), 52 / 55 (270,000), 27.0 / 26.7 (109,000), 10.2 / 9.5 (900);
-//   kNN lanes per query 1 / 2 / 4: 145 / 170 / 240 (668,000 supervoxels, K = 8),
-//     385 / 570 / 965 (4.9M one-voxel queries), 68 / 65 / 70 (200,000), 71 / 57 /
-//     52 (60,000, K = 8), 33 / 25.5 / 23 (25,000); a wave per query on the
-//     smallest batches: 6.2 against 16.5 with 2 lanes (900).
+//   kNN, a wave per query against 4 lanes: K = 5 0.84 / 0.88 (7,700 queries),
+//     0.904 / 0.901 (11,700), 0.93 / 0.87 (15,400), K = 8 1.00 / 1.06 (11,700),
+//     1.06 / 1.06 (15,400), 1.29 / 1.22 (23,300); 4 lanes against 2: K = 5 1.29 /
+//     1.33 (53,000), 1.65 / 1.62 (117,000); 2 against 1: 2.53 / 2.53 (263,000),
+//     K = 8 3.09 / 3.05; per launch 170 / 145 (668,000, K = 8). Blocks of 64 for
+//     4 lanes and 1: within 1% of 256, or up to 1.5% faster.
 Tiles tgmm::tiles_for(long long S, long long G, int K, bool voxel) {
   Tiles t = kDefaultTiles;
   if (S >= 6 * G)
@@ -239,7 +247,7 @@ Tiles tgmm::tiles_for(long long S, long long G, int K, bool voxel) {
     t.ll_gw = 64;
     t.ll_u = 2;
   }
-  if (S <= 16384) {
+  if (S <= (K <= 5 ? 12288 : 16384)) {
     t.knn_lanes = 64;
   } else if (S <= 65536) {
     t.knn_lanes = 4;
@@ -309,6 +317,7 @@ int batch_build(int device, const std::vector<FrameSrc>& fs_in, const tgmm_em_op
   std::vector<FrameDev> fh(fs.size());
   WsShape sh;
   long long v = 0, s = 0, g = 0, c = 0;
+  long long s_sum = 0, g_sum = 0;  // supervoxels and Gaussians without padding
   for (size_t i = 0; i < fs.size(); i++) {
     const FrameSrc& f = fs[i];
     if (f.N < 0 || f.S < 0 || f.G < 0) {
@@ -340,6 +349,8 @@ int batch_build(int device, const std::vector<FrameSrc>& fs_in, const tgmm_em_op
     s += round_up(std::max<long long>(f.S, 1), kAlign);
     g += round_up(f.G + 1, kAlign);
     c += F.ncap;
+    s_sum += f.S;
+    g_sum += f.G;
   }
   sh.Vcap = std::max<long long>(v, 1);
   sh.Scap = std::max<long long>(s, kAlign);
@@ -408,7 +419,7 @@ int batch_build(int device, const std::vector<FrameSrc>& fs_in, const tgmm_em_op
   P.Sext = need.Scap;
   P.Gext = need.Gcap;
   P.Cext = need.Ccap;
-  b->ko.tiles = tiles_for(s, g, o.K, o.voxel_mode != 0);
+  b->ko.tiles = tiles_for(s_sum, g_sum, o.K, o.voxel_mode != 0);
   int rc = batch_upload(b, fs);
   if (rc) {
     tgmm_batch_destroy(b);

@@ -433,7 +433,8 @@ extern "C" int tgmm_server_submit(tgmm_server* s, int stream_id, const tgmm_fram
 
 // Kernel grids cover the ranges allocated so far (high-water marks), not the
 // whole budget-sized workspace; the captured iteration is re-captured when
-// they grow.
+// they grow, with the launch shapes for the frames that hold ranges and can
+// run together (a stream's next frame waits for the one in flight).
 static int update_extents(tgmm_server* s) {
   DevPtrs& P = s->ws.P;
   const long long se = std::max<long long>(rup(s->as.high_water(), kAlign), kAlign);
@@ -443,8 +444,16 @@ static int update_extents(tgmm_server* s) {
   P.Sext = std::min(se, P.Scap);
   P.Gext = std::min(ge, P.Gcap);
   P.Cext = std::min(ce, P.Ccap);
-  if (!s->user_tiles)  // (knn_cell stays: the grids in flight were built with it)
-    s->ko.tiles = tiles_for(P.Sext, P.Gext, s->o.em.K, false);
+  if (!s->user_tiles) {  // (knn_cell stays: the grids in flight were built with it)
+    long long S = 0, G = 0;
+    for (const auto& kv : s->tickets) {
+      const Ticket& t = kv.second;
+      if (t.state != 1 && (t.state != 3 || (t.stream >= 0 && s->streams[t.stream].busy))) continue;
+      S += t.S;
+      G += t.G;
+    }
+    s->ko.tiles = tiles_for(S, G, s->o.em.K, false);
+  }
   if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
   if (s->graph) (void)hipGraphDestroy(s->graph);
   s->gexec = nullptr;
