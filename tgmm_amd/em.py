@@ -311,6 +311,12 @@ def pinned(a):
     return out
 
 
+# Raised when the kernels' fastest shapes change: a choice cached for other
+# kernels is not taken (with looks instead of whole searches, small grid cells
+# went from the fastest to the slowest at 60,000 Gaussians).
+_TILES_VERSION = 2
+
+
 def _tiles_cache_path():
     """Autotuner cache: $TGMM_TILES_CACHE, else ~/.cache/tgmm_amd/tiles.json."""
     return os.environ.get("TGMM_TILES_CACHE") or os.path.join(
@@ -667,9 +673,9 @@ class Batch:
     def autotune(self, reps=3, cache=True):
         """Pick the tile shapes by timing the candidates on this batch
         (tgmm_batch_autotune), or reuse the choice cached for the same
-        workload signature. Leaves the batch in its initial state. Returns
+        workload signature by the same version of the kernels' shapes. Leaves the batch in its initial state. Returns
         (tiles dict, report text or None when cached)."""
-        key = self.signature()
+        key = "t%d_%s" % (_TILES_VERSION, self.signature())
         path = _tiles_cache_path()
         table = {}
         if cache and os.path.exists(path):
