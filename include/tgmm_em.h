@@ -305,12 +305,16 @@ typedef struct tgmm_tiles {
 int tgmm_batch_set_tiles(tgmm_batch* b, const tgmm_tiles* tiles);
 int tgmm_batch_get_tiles(tgmm_batch* b, tgmm_tiles* tiles);
 /* Autotuner. For each knob in turn (log-likelihood shape, M-step lanes,
- * E-step block, kNN block) it times every candidate, the other knobs held at
- * the best so far, over `reps` eager iterations of the batch's own frames
- * from their initial state (hipEvents around the kernel on the batch
- * stream), and keeps the fastest. Leaves the batch in its initial state with
- * the chosen tiles. `chosen` and `report` (one line per candidate: knob,
- * shape, microseconds per launch) are optional. */
+ * E-step block, kNN cell size, kNN block and lanes) it times the candidates,
+ * the other knobs held at the best so far, on eager iterations of the batch's
+ * own frames from their initial state (hipEvents around the kernel on the
+ * batch stream), and keeps the fastest. The first three knobs take `reps`
+ * iterations. The two kNN knobs take a solve's (max_iter, at most 32) whatever
+ * `reps` is, since the search changes from whole to partial over a solve, and
+ * count all that the search launches. A candidate is dropped as soon as its
+ * time passes the best one's. Leaves the batch in its initial state with the
+ * chosen tiles. `chosen` and `report` (one line per candidate: knob, shape,
+ * microseconds per launch over the iterations run) are optional. */
 int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, char* report,
                         int report_cap);
 

@@ -832,8 +832,10 @@ extern "C" int tgmm_batch_get_tiles(tgmm_batch* b, tgmm_tiles* t) {
 }
 
 // Device time of one launch of kernel `tk`, averaged over `iters` eager
-// iterations from the initial state, with launch shapes `t`.
-static int time_shape(tgmm_batch* b, const Tiles& t, int tk, int iters, hipEvent_t e0,
+// iterations from the initial state, with launch shapes `t`; over those run
+// until their sum passed what `iters` launches of `best` ms take, if it did
+// (the average is above `best` then, whatever the rest would be).
+static int time_shape(tgmm_batch* b, const Tiles& t, int tk, int iters, double best, hipEvent_t e0,
                       hipEvent_t e1, double* ms_out) {
   KOpts ko = b->ko;
   ko.tiles = t;
@@ -841,14 +843,17 @@ static int time_shape(tgmm_batch* b, const Tiles& t, int tk, int iters, hipEvent
     if (int rc = regrid(b, ko)) return rc;
   if (int rc = tgmm_batch_reset(b)) return rc;
   double tot = 0.0;
-  for (int it = 0; it < iters; it++) {
+  int it = 0;
+  const double n = timed_launches(tk);
+  while (it < iters && tot <= best * n * iters) {
     HIPCHK(launch_iteration(b->ws.P, ko, b->st, e0, e1, tk));
     HIPCHK(hipEventSynchronize(e1));
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, e0, e1));
     tot += ms;
+    it++;
   }
-  *ms_out = tot / ((double)iters * timed_launches(tk));
+  *ms_out = tot / (it * n);
   return TGMM_OK;
 }
 
@@ -902,7 +907,7 @@ extern "C" int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, 
         t.ll_gw = 1;
         t.ll_u = 1;
         double ms = 0.0;
-        if ((rc = time_shape(b, t, kb.tk, iters, e0, e1, &ms)) != TGMM_OK) break;
+        if ((rc = time_shape(b, t, kb.tk, iters, tbest, e0, e1, &ms)) != TGMM_OK) break;
         snprintf(line, sizeof(line), "%s 1x1 %.2f\n", kb.name, 1000.0 * ms);
         rep += line;
         if (ms < tbest) {
@@ -923,7 +928,8 @@ extern "C" int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, 
           break;
       }
       double ms = 0.0;
-      if ((rc = time_shape(b, t, kb.tk, q >= 3 ? search_iters : iters, e0, e1, &ms)) != TGMM_OK)
+      if ((rc = time_shape(b, t, kb.tk, q >= 3 ? search_iters : iters, tbest, e0, e1, &ms)) !=
+          TGMM_OK)
         break;
       if (q == 4 && kb.v[c][2] == 0)
         snprintf(line, sizeof(line), "%s cell%d %.2f\n", kb.name, kb.v[c][0] / 64, 1000.0 * ms);
