@@ -321,9 +321,11 @@ int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, char* repor
 /* Average device time (ms) of one launch of the named kernel over `reps`
  * eager iterations, measured with hipEvents on the batch stream. In each
  * iteration the events bracket 8 back-to-back launches of "loglik" (it
- * writes only its block partials) and one launch of "estep", "knn" and
- * "mstep" (they update state that a repeated launch would read). Leaves the
- * state advanced. */
+ * writes only its block partials), one launch of "estep" and "mstep" and all
+ * that the search launches, "knn" (they update state that a repeated launch
+ * would read). bytes_per_launch: the bytes that a launch cannot do without;
+ * for "knn" the average over the iterations, which search for every query or
+ * for those whose neighbours may have changed. Leaves the state advanced. */
 int tgmm_batch_time_kernel(tgmm_batch* b, const char* name, int reps,
                            double* avg_ms, double* bytes_per_launch);
 int tgmm_batch_destroy(tgmm_batch* b);

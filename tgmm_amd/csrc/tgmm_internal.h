@@ -57,6 +57,8 @@ struct FrameDev {
                       // those of them it lists whatever moved
   int moved;          // means that moved since the last kNN search
   int blind;          // a look listed too many whatever moved: no more looks
+  int looked;         // the last iteration looked at the frame's queries,
+  int searched;       // and searched for this many (all, or those listed)
   int packed;         // every voxel's offset from its supervoxel's anchor is a
                       // small integer: the log-likelihood reads vpk (set to 1
                       // on the host, cleared by the moments kernel)
@@ -247,8 +249,8 @@ hipError_t launch_finalize(const DevPtrs& P, const KOpts& O, int cap, int only_f
                            int writeback, hipStream_t st);
 
 // timed_kernel ids for launch_iteration
-// (TK_SEARCH: the kNN search with what follows it, looks, searches again, ties)
-enum { TK_KNN = 0, TK_ESTEP = 1, TK_MSTEP = 2, TK_LOGLIK = 3, TK_SEARCH = 4 };
+// (TK_KNN: all that the search launches, looks, searches again, ties)
+enum { TK_KNN = 0, TK_ESTEP = 1, TK_MSTEP = 2, TK_LOGLIK = 3 };
 // launches between the timing events: the log-likelihood, which writes only
 // its block partials, runs kTimedLaunches times back to back, so the event
 // pair's own dispatch gap is spread over them; every other kernel updates

@@ -584,10 +584,25 @@ __device__ inline void scan_frame(const DevPtrs& P, const FrameDev* F, int which
   }
 }
 
+// The end of an iteration's search in frame f's state: what it did, whether it
+// looks again, and the counts of the next (k_iter_init has those of the first).
+__device__ inline void search_done(const DevPtrs& P, int f) {
+  FrameDev* F = P.fr + f;
+  if (f >= P.nframes || F->ncap == 0 || !F->active) return;
+  const unsigned long long again = F->again;
+  const bool looked = look_due(F->iter, F->blind, F->moved, F->ng);
+  const bool listed = looked && look_few((long long)(again & 0xffffffffull), F->ns);
+  F->looked = looked ? 1 : 0;
+  F->searched = listed ? (int)again : (int)F->ns;
+  if (look_futile((long long)(again >> 32), F->ns)) F->blind = 1;
+  F->moved = 0;
+  F->again = 0;
+}
+
 // Scan 0 follows the binning of the means for the next iteration (k_death,
 // k_gauss_prep). Blocks past the frames' (an iteration has them) form the
-// frames' sums of alpha, which wait for the same kernel and nothing else: one
-// launch instead of two. The search's grid (cell_start) still belongs to the
+// frames' sums of alpha, which wait for the same kernel and nothing else, and
+// close the search in another wave: one launch instead of two. The search's grid (cell_start) still belongs to the
 // last search, whose slot layout may yet be replayed, so the scan goes to
 // cell_next and k_grid_scatter takes it over.
 __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int need_active,
@@ -597,17 +612,13 @@ __global__ __launch_bounds__(1024) void k_scan_frames(DevPtrs P, int which, int 
   const int nscan = P.only_frame >= 0 ? 1 : P.nframes;
   if ((int)blockIdx.x >= nscan) {
     if (threadIdx.x < 64) alpha_sum_frame(P, (int)blockIdx.x - nscan, need_active);
+    if (threadIdx.x == 64) search_done(P, (int)blockIdx.x - nscan);
     return;
   }
   const int f = (P.only_frame >= 0) ? P.only_frame : (int)blockIdx.x;
   if (f >= P.Fcap || (P.only_frame < 0 && f >= P.nframes)) return;
   const FrameDev* F = P.fr + f;
   if (F->ncap == 0 || (need_active && !F->active)) return;  // empty slot / finished
-  if (which == 0 && threadIdx.x == 0) {
-    if (look_futile((long long)(F->again >> 32), F->ns)) P.fr[f].blind = 1;
-    P.fr[f].moved = 0;
-    P.fr[f].again = 0;
-  }
   const int* in;
   int* out;
   long long n;
@@ -1305,7 +1316,7 @@ __device__ inline bool knn_looks(const FrameDev* F) {
 // the frame whole after all. The look cannot clear a query whose K-th
 // neighbour lies outside its block of cells, and with many slots or few means
 // a cell those are many, however few means moved: where they alone are past
-// the line the frame's later iterations do not look (k_scan_frames, FrameDev's
+// the line the frame's later iterations do not look (search_done, FrameDev's
 // blind). 60,000 Gaussians, K = 8, 2 means a cell: 13.3 ms a solve, 14.7 with
 // a look in every iteration that is due one, 13.8 with none (6 a cell: 11.0).
 __device__ inline bool knn_listed(const FrameDev* F) {
@@ -3796,15 +3807,14 @@ static hipError_t iteration_t(const DevPtrs& P, const KOpts& O, hipStream_t st, 
   const unsigned gb = nb(P.Gext, kGB);
   const int bs = O.tiles.sv_block;
   k_grid_scatter<<<gb, kGB, 0, st>>>(P, O);
-  if ((tk == TK_KNN || tk == TK_SEARCH) && e0) (void)hipEventRecord(e0, st);
+  if (tk == TK_KNN && e0) (void)hipEventRecord(e0, st);
   launch_knn<KM>(P, O, st);
-  if (tk == TK_KNN && e1) (void)hipEventRecord(e1, st);
   {
     const int words = scan_words((int)std::min<long long>(kLayoutWords, (P.Gext + 63) / 64));
     k_knn_exact<KM><<<O.tiles.knn_lanes == 64 ? 128 : kFewBlocks, 64, scan_lds_bytes(words, false),
                       st>>>(P, O, words);
   }
-  if (tk == TK_SEARCH && e1) (void)hipEventRecord(e1, st);
+  if (tk == TK_KNN && e1) (void)hipEventRecord(e1, st);
   if (tk == TK_ESTEP && e0) (void)hipEventRecord(e0, st);
   k_estep<KM><<<nb(P.Sext, bs), bs, 0, st>>>(P, O);
   if (tk == TK_ESTEP && e1) (void)hipEventRecord(e1, st);

@@ -704,38 +704,52 @@ extern "C" int tgmm_batch_stats(tgmm_batch* b, tgmm_batch_stats_t* st) {
 }
 
 // Algorithmic bytes of one launch of a kernel over all frames of the batch
-// (compulsory traffic; Gaussian-side gathers counted once per Gaussian).
-static double kernel_bytes(tgmm_batch* b, int tk) {
+// (compulsory traffic; Gaussian-side gathers counted once per Gaussian), for
+// the iteration that the frame states fd were read after. In voxel mode the
+// supervoxels are the voxels (z.S = z.N).
+static double kernel_bytes(const tgmm_batch* b, int tk, const std::vector<FrameDev>& fd) {
   const int K = b->ws.K;
+  const bool voxel = b->ko.voxel != 0;
   double t = 0.0;
-  // whether each frame's voxels are read packed (decided on the device)
-  std::vector<FrameDev> fd(b->fh.size());
-  if (!fd.empty() &&
-      hipMemcpy(fd.data(), b->ws.P.fr, fd.size() * sizeof(FrameDev), hipMemcpyDeviceToHost) !=
-          hipSuccess)
-    fd.clear();
   for (size_t i = 0; i < b->sizes.size(); i++) {
     const auto& z = b->sizes[i];
     const double N = (double)z.N, S = (double)z.S, G = (double)z.G;
-    const bool packed = i < fd.size() && fd[i].packed != 0 && !b->ko.voxel;
     switch (tk) {
       case TK_LOGLIK:
-        // voxels (8 B packed, else 16 B); per supervoxel its frame, length,
-        // first voxel, anchor, ball and K candidates; a 64-byte pack per
-        // Gaussian
-        t += (packed ? 8.0 : 16.0) * N + S * (4 + 4 + 8 + 12 + 16 + 4.0 * K) + G * 64;
+        // voxels (8 B packed, as decided on the device, else 16 B); per
+        // supervoxel its frame, length, first voxel, anchor, ball and K
+        // candidates; a 64-byte pack per Gaussian. A lane per voxel reads
+        // its frame, anchor, intensity and candidates.
+        if (voxel && b->ko.tiles.ll_gw == 1)
+          t += S * (4 + 12 + 4 + 4.0 * K) + G * sizeof(LLPack);
+        else
+          t += (fd[i].packed != 0 && !voxel ? 8.0 : 16.0) * N +
+               S * (4 + 4 + 8 + 12 + 16 + 4.0 * K) + G * sizeof(LLPack);
         break;
       case TK_ESTEP:
-        t += S * (4 + 80 + 4.0 * K + 4.0 * K) + G * (8 * 11);
+        // per supervoxel its frame, 10 moments (a voxel: its anchor and
+        // intensity), K candidates in and K responsibilities out
+        t += S * (4 + (voxel ? 16 : 80) + 4.0 * K + 4.0 * K) + G * sizeof(EPack);
         break;
-      case TK_KNN:
-        // per query its centroid and index (16 B), the previous candidates
-        // (the bound) and the new ones (4 B each); per Gaussian its binned
-        // reference and its mean for the bound (16 B each)
-        t += S * (16 + 8.0 * K) + G * 32;
+      case TK_KNN: {
+        // per query searched for its centroid and index (16 B), the previous
+        // candidates (the bound) and the new ones (4 B each); per Gaussian,
+        // where the frame is searched whole, its binned reference and its mean
+        // for the bound (16 B each); per query looked at what its last search
+        // left and its cell. A wave per query looks by itself: what it
+        // searches for after the first iteration is not counted.
+        const bool own = b->ko.tiles.knn_lanes == 64;
+        const bool whole = own ? fd[i].iter <= 2 : fd[i].searched == z.S;
+        t += (whole ? S : own ? 0.0 : (double)fd[i].searched) * (16 + 8.0 * K);
+        t += whole ? G * 32 : 0.0;
+        t += (own ? !whole : fd[i].looked != 0) ? S * 8 : 0.0;
         break;
+      }
       case TK_MSTEP:
-        t += G * (27 * 8 * 2 + 8) + S * (4 + 4 + 80);
+        // per Gaussian its mean, alpha, flags and list bounds, and 10 sums out;
+        // per supervoxel a pair, its responsibility and 10 moments (a voxel:
+        // its anchor)
+        t += G * (24 + 8 + 8 + 1 + 4 + 80) + S * (4 + 4 + (voxel ? 12 : 80));
         break;
     }
   }
@@ -760,7 +774,8 @@ extern "C" int tgmm_batch_time_kernel(tgmm_batch* b, const char* name, int reps,
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   // eager iterations from the initial state; `reps` launches of the kernel
-  double tot = 0.0;
+  double tot = 0.0, bytes = 0.0;
+  std::vector<FrameDev> fd(b->fh.size());
   int it = b->opts.max_iter;
   for (int r = 0; r < reps; r++) {
     if (it == b->opts.max_iter) {
@@ -773,11 +788,17 @@ extern "C" int tgmm_batch_time_kernel(tgmm_batch* b, const char* name, int reps,
     HIPCHK(hipEventElapsedTime(&ms, e0, e1));
     tot += ms;
     it++;
+    if (bytes_per_launch && (tk == TK_KNN || r == 0)) {  // the others' stay the same
+      HIPCHK(hipMemcpyAsync(fd.data(), b->ws.P.fr, fd.size() * sizeof(FrameDev),
+                            hipMemcpyDeviceToHost, b->st));
+      HIPCHK(hipStreamSynchronize(b->st));
+      bytes += kernel_bytes(b, tk, fd);
+    }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   *avg_ms = tot / ((double)reps * timed_launches(tk));
-  if (bytes_per_launch) *bytes_per_launch = kernel_bytes(b, tk);
+  if (bytes_per_launch) *bytes_per_launch = tk == TK_KNN ? bytes / reps : bytes;
   return TGMM_OK;
 }
 
@@ -884,8 +905,8 @@ extern "C" int tgmm_batch_autotune(tgmm_batch* b, int reps, tgmm_tiles* chosen, 
                                  {64, 1}, {64, 2}, {64, 4}}},
       {"mstep", TK_MSTEP, 3, {{4, 0}, {8, 0}, {16, 0}}},
       {"estep", TK_ESTEP, 3, {{64, 0}, {128, 0}, {256, 0}}},
-      {"knn_cell", TK_SEARCH, 3, {{2, 0}, {4, 0}, {6, 0}}},
-      {"knn", TK_SEARCH, 15, {{64, 8, 0},  {128, 8, 0}, {256, 8, 0}, {64, 4, 1},  {256, 4, 1},
+      {"knn_cell", TK_KNN, 3, {{2, 0}, {4, 0}, {6, 0}}},
+      {"knn", TK_KNN, 15, {{64, 8, 0},  {128, 8, 0}, {256, 8, 0}, {64, 4, 1},  {256, 4, 1},
                            {64, 8, 1},  {256, 8, 1}, {64, 4, 2},  {256, 4, 2}, {64, 8, 2},
                            {256, 8, 2}, {64, 4, 4},  {256, small ? 8 : 4, small ? 64 : 4}, {64, 8, 4},
                            {256, 8, 4}}},
