@@ -129,7 +129,8 @@ struct DevPtrs {
   long long* sv_beg;
   int* sv_len;
   float* sv_cent;   // 3*Scap SoA
-  double* mom;      // 10*Scap: n, c[3], Q[6]  (unweighted, FP64)
+  double* mom;      // 10*Scap: n, c[3], Q[6]  (unweighted, FP64; this and wmom not
+                    // in voxel mode)
   double* wmom;     // 10*Scap: W, mu[3], C[6] (intensity-weighted, FP64), the 10 values
                     // of a supervoxel contiguous (wmom[10 s + i]: one M-step pair reads
                     // 80 bytes in a row)

@@ -267,8 +267,9 @@ __global__ __launch_bounds__(256) void k_moments(DevPtrs P) {
 }
 
 // Voxel mode: every supervoxel is one voxel, so its moments are the voxel
-// itself (count 1, mean x, no scatter) and its M-step weight is the stored
-// responsibility, which already carries the intensity (GMEM.cu:2216-2222).
+// itself (count 1, mean x, no scatter), which the iteration's kernels take from
+// the anchor, and its M-step weight is the stored responsibility, which already
+// carries the intensity (GMEM.cu:2216-2222).
 __global__ __launch_bounds__(256) void k_moments_voxel(DevPtrs P) {
   const long long s = P.s_lo + (long long)blockIdx.x * 256 + threadIdx.x;
   if (s >= P.Scap) return;
@@ -276,19 +277,8 @@ __global__ __launch_bounds__(256) void k_moments_voxel(DevPtrs P) {
   if (f < 0 || (P.only_frame >= 0 && f != P.only_frame)) return;
   const long long S = P.Scap, v = P.sv_beg[s];
   const float x[3] = {P.vx[v], P.vy[v], P.vz[v]};
-  P.mom[s] = 1.0;
-  P.wmom[s * 10] = 1.0;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    P.mom[(1 + a) * S + s] = (double)x[a];
-    P.wmom[s * 10 + 1 + a] = (double)x[a];
-    P.anchor[a * S + s] = x[a];
-  }
-#pragma unroll
-  for (int i = 4; i < 10; i++) {
-    P.mom[i * S + s] = 0.0;
-    P.wmom[s * 10 + i] = 0.0;
-  }
+  for (int a = 0; a < 3; a++) P.anchor[a * S + s] = x[a];
   P.sv_ball[s] = make_float4(0.f, 0.f, 0.f, 0.f);
   // the voxel is its own anchor: offsets 0, unless a coordinate is not finite
   P.vpk[v] = make_int2((int)((unsigned)(s & 255) << 24), __float_as_int(P.vimg[v]));
