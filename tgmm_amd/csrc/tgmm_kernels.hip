@@ -1628,7 +1628,10 @@ using SlotsOf = typename std::conditional<ONE, ScanSlotsOne<KM>, ScanSlots<KM>>:
 // search (mknn, in index order, and its grid), in one of two shapes:
 //   ONE = false: one query per lane (dead lanes take nothing); the Gaussians
 //     are loaded 64 at a time (one a lane), and those inside the box of the
-//     wave's balls (below) are broadcast to the lanes in index order;
+//     wave's balls (below) go through every lane's scan in index order: with
+//     up to 5 slots they are collected in LDS and each lane walks those it
+//     marked (scan_marked), with more they are broadcast one after another
+//     (scan_each);
 //   ONE = true: the wave's single query (every lane holds it); 64 Gaussians
 //     are tested at once (one a lane) and the sequential rule is applied to
 //     the lanes that pass the current threshold, lowest index first, the
@@ -1651,7 +1654,8 @@ using SlotsOf = typename std::conditional<ONE, ScanSlotsOne<KM>, ScanSlots<KM>>:
 //     LDS bitmap, compacted in index order into an LDS list, and scanned.
 //     When the box or the bitmap is too large (no box yet, or more Gaussians
 //     than the bitmap holds), every later Gaussian is scanned.
-// LDS: words_cap bitmap words, then kListCap list entries.
+// LDS: words_cap bitmap words, then kListCap list entries, then (marking only)
+// 64 * (kScanU + 1) collected Gaussians.
 constexpr int kLayoutCells = 8192;  // most grid cells marked per wave
 constexpr int kLayoutWords = 4096;  // largest bitmap (Gaussians / 64) in LDS: 32 KiB
 constexpr int kListCap = 1024;      // marked Gaussians listed at a time
@@ -3469,8 +3473,9 @@ __global__ __launch_bounds__(NT) void k_loglik(DevPtrs P, KOpts O) {
 // by its loads: the candidates' indices and packs, and 20 bytes a voxel (the
 // anchor, the intensity, the frame); reading the voxel's coordinates, range
 // and length as well, for the same terms, took 114 us instead of 77 on 4.9M
-// voxels. (With the anchor the voxel, U (x - a) is 0, or not finite where e is
-// not either, and such a term is dropped.)
+// voxels. (With the anchor the voxel, U (x - a) is 0 for a finite U. A
+// coordinate that is not finite makes e not finite, and the term is dropped;
+// with an entry of U past float's range, nu W above 1e76, e alone decides.)
 template <int KM>
 __global__ __launch_bounds__(256) void k_loglik_voxel(DevPtrs P, KOpts O) {
   __shared__ double tree[256];

@@ -55,8 +55,8 @@ __device__ inline unsigned long long div_exact(unsigned long long n, unsigned lo
   return q;
 }
 
-// The same in 32 bits, for n < 2^32 and d < 2^32: the double product is exact
-// The same for n and d below 2^32.
+// The same for n and d below 2^32: the truncated product is off by at most one
+// there too, and the remainder fixes it.
 __device__ inline unsigned div_exact32(unsigned n, unsigned d, double inv, unsigned& r) {
   unsigned q = (unsigned)((double)n * inv);
   long long rem = (long long)n - (long long)((unsigned long long)q * d);
