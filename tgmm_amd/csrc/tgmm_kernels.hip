@@ -925,10 +925,9 @@ __device__ inline float* knn_left(const DevPtrs& P, long long i) {
 // keeps is searched again.
 // In the EM's later iterations most means do not move at all in f32 (frame of
 // 60,000 Gaussians: 1% move in the 7th iteration, 0.1% in the 12th).
-__device__ inline bool knn_needed(float kd, const int* qcell, const int* cell_mv,
-                                  const float4* mv_pos, const float4* q4, const FrameDev* F,
-                                  float s0, float s1, float s2, long long i) {
-  const int cell = qcell[i];
+__device__ inline bool knn_needed(float kd, int cell, const int* cell_mv, const float4* mv_pos,
+                                  const float4* q4, const FrameDev* F, float s0, float s1,
+                                  float s2, long long i) {
   if (!(kd >= 0.0f)) return true;
   const int nx = F->dims[0], ny = F->dims[1], nz = F->dims[2];
   const long long c0 = F->c0;
@@ -1325,8 +1324,10 @@ __global__ __launch_bounds__(256) void k_knn_look(DevPtrs P, KOpts O) {
   const FrameDev* F = P.fr + f;
   if (!knn_looks(F)) return;
   const bool in = i < F->s0 + F->ns;
-  const float kd = in ? *knn_left(P, i) : 0.0f;
-  const bool need = in && knn_needed(kd, P.qcell, P.cell_mv, P.mv_pos, P.q4, F, O.scale[0],
+  // in one round of loads, also past the frame's last query (i < Scap)
+  const float kd = *knn_left(P, i);
+  const int cell = P.qcell[i];
+  const bool need = in && knn_needed(kd, cell, P.cell_mv, P.mv_pos, P.q4, F, O.scale[0],
                                      O.scale[1], O.scale[2], i);
   const unsigned long long m = __ballot(need), stuck = __ballot(in && !(kd >= 0.0f));
   if (m == 0ull) return;
@@ -1371,7 +1372,7 @@ __global__ __launch_bounds__(256) void k_knn_small(DevPtrs P, KOpts O) {
   if (f < 0 || !P.fr[f].active) return;
   const FrameDev* F = P.fr + f;
   if (i >= F->s0 + F->ns) return;  // whole waves
-  if (F->iter > 1 && !knn_needed(*knn_left(P, i), P.qcell, P.cell_mv, P.mv_pos, P.q4, F,
+  if (F->iter > 1 && !knn_needed(*knn_left(P, i), P.qcell[i], P.cell_mv, P.mv_pos, P.q4, F,
                                  O.scale[0], O.scale[1], O.scale[2], i))
     return;
   const bool tie = knn_wave<KM>(P, O, F, i, rows[w]);
@@ -2512,7 +2513,7 @@ __global__ __launch_bounds__(256) void k_pair_scatter(DevPtrs P, KOpts O) {
 // pair scan): up to kRunLds runs ranked in LDS, a run a thread; beyond, the
 // pairs laid out and sorted in LDS (bitonic), or, past kSortLds pairs, the
 // runs ranked against all of them, kRunTile at a time through LDS, eight a
-// thread (four lists of 20,000 single-pair runs: 8 ms an iteration; with each
+// thread (four lists of 20,000 single-pair runs: 9 ms an iteration; with each
 // comparison's code and length read from memory 103, with only the codes of
 // the pairs 96).
 // Both sides read the run count; whichever handles a Gaussian clears it (the
@@ -2591,6 +2592,46 @@ __device__ inline void seg_sort_short(const DevPtrs& P, int* sh) {
   }
 }
 
+// The runs of one list ranked against each other, kRunTile at a time through
+// LDS (tile, free again at the end), and their pairs written out, by a block.
+// Not inlined: inside the kernel it made every iteration of the usual lists
+// 0.25 us longer (10,000 Gaussians).
+__device__ __noinline__ void rank_runs(const int* __restrict__ first,
+                                       const unsigned char* __restrict__ len,
+                                       int* __restrict__ sorted, int nr, int2* tile) {
+  constexpr int R = 8;  // runs a thread ranks at once
+  const int t = threadIdx.x;
+  for (int r0 = 0; r0 < nr; r0 += 256 * R) {
+    int c[R], at[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const int r = r0 + t + 256 * q;
+      c[q] = r < nr ? first[r] : INT_MIN;
+      at[q] = 0;
+    }
+    for (int b = 0; b < nr; b += kRunTile) {
+      const int m = min(kRunTile, nr - b);
+      __syncthreads();  // the tile before has been read
+      for (int i = t; i < m; i += 256) tile[i] = make_int2(first[b + i], len[b + i]);
+      __syncthreads();
+#pragma unroll 4
+      for (int i = 0; i < m; i++) {
+        const int2 v = tile[i];
+#pragma unroll
+        for (int q = 0; q < R; q++) at[q] += v.x < c[q] ? v.y : 0;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const int r = r0 + t + 256 * q;
+      if (r >= nr) continue;
+      const int n = len[r];
+      for (int u = 0; u < n; u++) sorted[at[q] + u] = c[q] + (u << kPairShift);
+    }
+  }
+  __syncthreads();  // every thread has read the tile
+}
+
 __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int nlong) {
   __shared__ int fill;
   const int cnt = P.knn_ctl[2];
@@ -2635,38 +2676,8 @@ __device__ inline void seg_sort_long(const DevPtrs& P, int* sh, int first, int n
       continue;
     }
     if (L > kSortLds) {
-      constexpr int R = 8;  // runs a thread ranks at once
-      int2* tile = reinterpret_cast<int2*>(sh);
-      for (int r0 = 0; r0 < nr; r0 += 256 * R) {
-        int c[R], at[R];
-#pragma unroll
-        for (int q = 0; q < R; q++) {
-          const int r = r0 + t + 256 * q;
-          c[q] = r < nr ? P.pairs[st + r] : INT_MIN;
-          at[q] = 0;
-        }
-        for (int b = 0; b < nr; b += kRunTile) {
-          const int m = min(kRunTile, nr - b);
-          __syncthreads();  // the tile before has been read
-          for (int i = t; i < m; i += 256)
-            tile[i] = make_int2(P.pairs[st + b + i], P.run_len[st + b + i]);
-          __syncthreads();
-#pragma unroll 4
-          for (int i = 0; i < m; i++) {
-            const int2 v = tile[i];
-#pragma unroll
-            for (int q = 0; q < R; q++) at[q] += v.x < c[q] ? v.y : 0;
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < R; q++) {
-          const int r = r0 + t + 256 * q;
-          if (r >= nr) continue;
-          const int n = P.run_len[st + r];
-          for (int u = 0; u < n; u++) P.pairs_sorted[st + at[q] + u] = c[q] + (u << kPairShift);
-        }
-      }
-      __syncthreads();  // every thread has read the count, and sh is free
+      rank_runs(P.pairs + st, P.run_len + st, P.pairs_sorted + st, nr,
+                reinterpret_cast<int2*>(sh));
       if (t == 0) P.run_cnt[k] = 0;
       continue;
     }
