@@ -252,8 +252,9 @@ static int server_capture(tgmm_server* s) {
 
 // Capacity from the budget: supervoxels >= 8 voxels and Gaussians >= 32 voxels
 // on average, two grid cells per Gaussian plus slack per slot. A power of two
-// of voxels, at least 2^20; where the last doubling is up to a sixteenth above
-// the budget, it is taken and trimmed to fit instead of left out.
+// of voxels, at least 2^20; where the last doubling is up to 1/22 above the
+// budget, it is taken and trimmed to fit instead of left out (a sum of element
+// sizes, by which budgets were once matched, was 2.7 to 4.2% short of the arrays).
 WsShape server_shape(long long budget, int max_frames, int K) {
   auto shape = [&](long long V) {
     WsShape t;
@@ -266,7 +267,7 @@ WsShape server_shape(long long budget, int max_frames, int K) {
   };
   constexpr long long kLeast = 1LL << 20;
   long long V = kLeast;
-  while (2 * V <= (1LL << 31) && ws_bytes(shape(2 * V), K) - budget / 16 <= budget) V *= 2;
+  while (2 * V <= (1LL << 31) && ws_bytes(shape(2 * V), K) - budget / 22 <= budget) V *= 2;
   for (const long long step = V / 128; V > kLeast && ws_bytes(shape(V), K) > budget;) V -= step;
   return shape(V);
 }
