@@ -256,11 +256,15 @@ static int server_capture(tgmm_server* s) {
 // budget, it is taken and trimmed to fit instead of left out (a sum of element
 // sizes, by which budgets were once matched, was 2.7 to 4.2% short of the arrays).
 WsShape server_shape(long long budget, int max_frames, int K) {
+  // pair codes and slot positions are 32-bit (as a batch's placement checks):
+  // a large budget's supervoxels stop there
+  const long long lim = (1LL << 31) - 1;
+  const long long smax = std::min(lim >> kPairShift, lim / K) / kAlign * kAlign;
   auto shape = [&](long long V) {
     WsShape t;
     t.Fcap = max_frames;
     t.Vcap = V;
-    t.Scap = rup(V / 8 + 256LL * t.Fcap, kAlign);
+    t.Scap = std::min(rup(V / 8 + 256LL * t.Fcap, kAlign), smax);
     t.Gcap = rup(V / 32 + 256LL * t.Fcap, kAlign);
     t.Ccap = rup(t.Gcap / 2 + 2LL * kCB * t.Fcap, kCB);
     return t;
